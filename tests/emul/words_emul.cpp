@@ -1,0 +1,232 @@
+// Host run of the word-band logic (viennals_amd/csrc/lsg_words.hpp): one
+// operation through words, point masks and neighbour references as the word
+// kernels use them, lane by lane, on an EBand of lsg_emul.cpp.
+#include "lsg_emul.cpp"
+
+#include "../../viennals_amd/csrc/lsg_words.hpp"
+
+namespace {
+
+struct Words {
+  Frame f;
+  GridInfo g;
+  std::vector<WordBits> wb;
+  std::vector<double> val;
+  Words(const Frame &f_, const GridInfo &g_) : f(f_), g(g_), wb(f_.nwords + 1, WordBits{0, 0}), val(64 * (f_.nwords + 1), 7e77) {}
+  WordView view() const { return WordView{wb.data(), val.data(), f, g}; }
+  void put(uint32_t w, int bit, double v) {
+    if (v < 0) wb[w].neg |= 1ull << bit;
+    if (!isUndef(v)) wb[w].def |= 1ull << bit;
+    val[((size_t)w << 6) | (uint32_t)bit] = v;
+  }
+};
+
+uint64_t validOf(const Frame &f, uint32_t w) {
+  int32_t kw, yr, zr;
+  f.wordRow(w, kw, yr, zr);
+  return wordValid(f, kw);
+}
+
+Words toWords(const EBand &d) {
+  Words o(d.f, d.g);
+  const uint32_t nw = (uint32_t)d.f.nwords;
+  if (d.f.base) o.put(nw, 0, d.val[0]);
+  for (uint32_t w = 0; w < nw; ++w)
+    for (int b = 0; b < 64; ++b) {
+      if (!(validOf(d.f, w) >> b & 1)) continue;
+      const double v = runValueAt(d.val.data(), d.bits[w], (uint32_t)d.f.base + d.pre[w], b);
+      check((d.bits[w] >> b & 1) || isUndef(v), "run of defined points");
+      o.put(w, b, v);
+    }
+  return o;
+}
+
+EBand toBand(const Words &o, const EBand &like, int width) {
+  EBand d;
+  d.D = like.D;
+  d.g = o.g;
+  d.f = o.f;
+  d.width = width;
+  const uint32_t nw = (uint32_t)o.f.nwords;
+  const WordView v = o.view();
+  d.bits.assign(nw + 1, 0);
+  d.pre.assign(nw + 1, 0);
+  if (o.f.base) {
+    d.val.push_back(v.point(nw, 0));
+    d.pos.push_back(POS_NONE);
+  }
+  uint32_t acc = 0;
+  for (uint32_t w = 0; w < nw; ++w) {
+    d.bits[w] = startsOfWord(o.wb.data(), o.f, w);
+    d.pre[w] = acc;
+    for (int b = 0; b < 64; ++b)
+      if (d.bits[w] >> b & 1) {
+        d.val.push_back(v.point(w, b));
+        d.pos.push_back((w << 6) | (uint32_t)b);
+        ++acc;
+      }
+  }
+  d.pre[nw] = acc;
+  return d;
+}
+
+double updated(const Words &in, uint32_t w, int bit, const double *rates, double dt, bool upd) {
+  const double v = in.view().point(w, bit);
+  return upd ? ruleUpdate(v, dt, isUndef(v) ? 0. : rates[((size_t)w << 6) | (uint32_t)bit]) : v;
+}
+
+bool g_conflict = false;
+
+template <int D, int OP>
+Words wordOp(const Words &in, double a, double b, const double *rates, double dt) {
+  Words o(in.f, in.g);
+  const Frame &f = in.f;
+  WordFrame F;
+  F.init(in.f, in.g);
+  const uint32_t nw = (uint32_t)f.nwords;
+  const bool star = OP == W_EXPAND || OP == W_REBUILD || OP == W_UPD_REBUILD, upd = OP == W_UPD_REBUILD;
+  g_conflict = false;
+  if (f.base) {
+    double c;
+    const double v = wordRuleMin<D, OP>(F, in.wb.data(), in.val.data(), rates, dt, a, b, c);
+    const double g = wordRuleAt<D, OP>(in.view(), in.g.lo, rates, dt, a, b);
+    check(std::memcmp(&v, &g, 8) == 0 && c == in.view().point(nw, 0), "grid-minimum star");
+    if (OP == W_EXPAND && isUndef(c) && v != c) g_conflict = true;
+    o.put(nw, 0, v);
+  }
+  for (uint32_t w = 0; w < nw; ++w) {
+    WordSite<D> site;
+    wordSite<D>(in.wb.data(), F, w, site);
+    const int32_t kw = site.kw, yr = site.yr, zr = site.zr;
+    const WordBits self = site.self;
+    if (star && quietSite<D>(F, site)) {
+      bool conflict = false;
+      check(starPoints<D, true>(in.wb.data(), F, w, site, conflict) == 0 && !conflict, "a quiet word has work");
+    }
+    const uint64_t cand = star ? starPoints<D, OP == W_EXPAND>(in.wb.data(), F, w, site, g_conflict) : self.def;
+    if (!cand) {
+      check(self.def == 0, "a defined point is left out");
+      o.wb[w] = self;
+      continue;
+    }
+    const int top = kw == wordLast(f) ? rowLastBit(f) : 63;
+    for (int lane = 0; lane < 64; ++lane) {
+      if (!(wordValid(f, kw) >> lane & 1)) continue;
+      const double c = updated(in, w, lane, rates, dt, upd);
+      if (!(cand >> lane & 1)) {
+        check(isUndef(c), "a defined point is left out");
+        o.put(w, lane, c);
+        continue;
+      }
+      auto at = [&](const WordRef &r) {
+        check(r.w <= nw && r.bit < 64, "reference out of range");
+        return updated(in, r.w, r.bit < 0 ? lane : r.bit, rates, dt, upd);
+      };
+      double nb[2 * D];
+      for (int d = 1; d < D; ++d) {
+        nb[d] = at(site.ref[2 * d - 2]);
+        nb[D + d] = at(site.ref[2 * d - 1]);
+      }
+      nb[0] = lane == top ? at(site.above) : updated(in, w, lane + 1, rates, dt, upd);
+      nb[D] = lane == 0 ? at(site.below) : updated(in, w, lane - 1, rates, dt, upd);
+      const double v = wordRule<D, OP>(c, nb, a, b);
+      int32_t p[3] = {kw * 64 + lane + f.o[0], yr + f.o[1], zr + f.o[2]};
+      const double g = wordRuleAt<D, OP>(in.view(), p, rates, dt, a, b);
+      check(std::memcmp(&v, &g, 8) == 0, "word neighbours differ from general lookups");
+      o.put(w, lane, v);
+    }
+  }
+  return o;
+}
+
+template <int D> Words runOp(const Words &in, int op, double a, double b, const double *rates, double dt) {
+  switch (op) {
+  case W_EXPAND: return wordOp<D, W_EXPAND>(in, a, b, rates, dt);
+  case W_REBUILD: return wordOp<D, W_REBUILD>(in, a, b, rates, dt);
+  case W_UPD_REBUILD: return wordOp<D, W_UPD_REBUILD>(in, a, b, rates, dt);
+  case W_REDUCE: return wordOp<D, W_REDUCE>(in, a, b, rates, dt);
+  case W_PRUNE: return wordOp<D, W_PRUNE>(in, a, b, rates, dt);
+  default: return wordOp<D, W_PRUNE_RSZ>(in, a, b, rates, dt);
+  }
+}
+
+// The same operation on the run list; list rates from slot rates.
+template <int D> EBand listOp(const EBand &in, int op, double a, double b, const double *rates, double dt) {
+  OpParams p{};
+  p.a = a;
+  p.b = b;
+  if (op == W_EXPAND || op == W_REBUILD) {
+    p.kind = op == W_EXPAND ? OP_EXPAND : OP_REBUILD;
+    return starOp<D>(in, p);
+  }
+  if (op == W_UPD_REBUILD) {
+    std::vector<double> r(in.val.size(), 0.);
+    for (size_t i = 0; i < r.size(); ++i)
+      if (in.pos[i] != POS_NONE) r[i] = rates[in.pos[i]];
+    return updRebuildOp<D>(in, r, dt, a);
+  }
+  p.kind = op == W_REDUCE ? OP_REDUCE : op == W_PRUNE ? OP_PRUNE : OP_PRUNE_RSZ;
+  return selfOp<D>(in, p, nullptr, 0.);
+}
+
+bool same(const EBand &x, const EBand &y) {
+  return x.pos == y.pos && x.bits == y.bits && x.pre == y.pre && x.val.size() == y.val.size() &&
+         std::memcmp(x.val.data(), y.val.data(), 8 * x.val.size()) == 0;
+}
+
+}  // namespace
+
+extern "C" {
+
+// Runs operation `op` on the band of `h` both ways; 0 when the results are
+// the same bit for bit, 1 when not, 3 when not but a conflict was reported, -1
+// on a failed check.  `rates`: one value
+// per frame position (null: none); the number of positions comes back from a
+// call with op = -1.
+int64_t emu_words_compare(void *h, int op, double a, double b, const double *rates, double dt) {
+  EBand &d = *(EBand *)h;
+  if (op < 0) return 64 * (d.f.nwords + 1);
+  const bool tiled = g_tiled;
+  g_tiled = false;
+  int64_t r = -1;
+  try {
+    const Words in = toWords(d);
+    if (!same(toBand(in, d, d.width), d)) r = 2;
+    else if (d.D == 2) r = same(toBand(runOp<2>(in, op, a, b, rates, dt), d, 0), listOp<2>(d, op, a, b, rates, dt)) ? 0 : 1;
+    else r = same(toBand(runOp<3>(in, op, a, b, rates, dt), d, 0), listOp<3>(d, op, a, b, rates, dt)) ? 0 : 1;
+    if (r == 1 && g_conflict) r = 3;
+  } catch (const std::exception &e) {
+    fprintf(stderr, "words_emul: %s\n", e.what());
+  }
+  g_tiled = tiled;
+  return r;
+}
+
+// Two bands on one frame through a boolean of kind `kind`.
+int64_t emu_words_boolean(void *ha, void *hb, int kind, double wT, double wS) {
+  EBand &A = *(EBand *)ha, &B = *(EBand *)hb;
+  if (std::memcmp(&A.f, &B.f, sizeof(Frame))) return -2;
+  const bool tiled = g_tiled;
+  g_tiled = false;
+  int64_t r = -1;
+  try {
+    const Words x = toWords(A), y = toWords(B);
+    Words o(A.f, A.g);
+    const uint32_t nw = (uint32_t)A.f.nwords;
+    for (uint32_t w = 0; w <= nw; ++w) {
+      if (!(x.wb[w].def | y.wb[w].def)) {
+        o.wb[w] = WordBits{0, boolNeg(kind, x.wb[w].neg, y.wb[w].neg)};
+        continue;
+      }
+      const uint64_t ok = w < nw ? validOf(A.f, w) : 1ull;
+      for (int b = 0; b < 64; ++b)
+        if (ok >> b & 1) o.put(w, b, ruleBoolean(kind, x.view().point(w, b), y.view().point(w, b), wT, wS));
+    }
+    r = same(toBand(o, A, 0), booleanOp(A, B, kind, wT, wS)) ? 0 : 1;
+  } catch (const std::exception &e) {
+    fprintf(stderr, "words_emul: %s\n", e.what());
+  }
+  g_tiled = tiled;
+  return r;
+}
+}

@@ -36,6 +36,8 @@ namespace lsg {
 
 #ifdef LSG_HOST_ONLY
 using std::fabs;
+using std::fmax;
+using std::fmin;
 using std::signbit;
 using std::sqrt;
 #endif

@@ -24,6 +24,7 @@
 #include "lsg_geometry.hpp"
 #include "lsg_kernels.hpp"
 #include "lsg_learned.hpp"
+#include "lsg_words_launch.hpp"
 
 namespace lsg {
 
@@ -158,6 +159,105 @@ struct WsStore {
   }
 };
 
+// Storage of a word band.
+struct WordStore {
+  WordBufs b;
+  int64_t nwAlloc = 0;
+  void release() {
+    if (b.wb) (void)hipFree(b.wb);
+    if (b.val) (void)hipFree(b.val - 64 * WORD_PAGES);
+    b = WordBufs{};
+    nwAlloc = 0;
+  }
+  int ensure(int64_t nw) {
+    if (b.wb && nwAlloc >= nw) return 0;
+    if (b.wb) LSG_HIP(hipStreamSynchronize(g_ctx.s));
+    release();
+    // sizes in steps of an eighth, so that bands of similar frames can be exchanged
+    int64_t step = 1024;
+    while (step * 16 <= nw) step *= 2;
+    nw = (nw + step - 1) / step * step;
+    LSG_HIP(hipMalloc(&b.wb, (nw + 1) * sizeof(WordBits)));
+    double *pages = nullptr;
+    LSG_HIP(hipMalloc(&pages, (nw + 1 + WORD_PAGES) * 64 * sizeof(double)));
+    launchWordPages(g_ctx.s, pages);
+    b.val = pages + 64 * WORD_PAGES;
+    nwAlloc = nw;
+    return 0;
+  }
+};
+
+// Bands between the operations of a step or of a call, the expanded starting
+// band of a Runge-Kutta step and the rates: one set for the process (every
+// call of the library runs on its one stream), as large as the largest frame
+// in use, freed with the last level set.
+struct WordWs {
+  WordStore w[2], init;
+  double *rates = nullptr;
+  uint64_t *act = nullptr;  // active points of the band whose rates are computed
+  int64_t ratesNw = 0;
+  double *box = nullptr;  // box alphas of the local Lax-Friedrichs scheme
+  size_t boxSlots = 0;
+  WordStep *st = nullptr;
+  int ensureOps(int64_t nw) {
+    for (WordStore &x : w)
+      if (int e = x.ensure(nw)) return e;
+    if (!st) {
+      LSG_HIP(hipMalloc(&st, sizeof(WordStep)));
+      LSG_HIP(hipMemset(st, 0, sizeof(WordStep)));
+    }
+    return 0;
+  }
+  int ensureBox(int64_t nw, int D) {
+    const size_t n = (size_t)(nw + 1) * 64 * D;
+    if (boxSlots >= n) return 0;
+    if (box) {
+      LSG_HIP(hipStreamSynchronize(g_ctx.s));
+      (void)hipFree(box);
+      box = nullptr;
+      boxSlots = 0;
+    }
+    LSG_HIP(hipMalloc(&box, n * sizeof(double)));
+    boxSlots = n;
+    return 0;
+  }
+  int ensureStep(int64_t nw, bool rungeKutta) {
+    if (int e = ensureOps(nw)) return e;
+    if (rungeKutta)
+      if (int e = init.ensure(nw)) return e;
+    if (!rates || ratesNw < nw) {
+      if (rates) {
+        LSG_HIP(hipStreamSynchronize(g_ctx.s));
+        (void)hipFree(rates - 64 * WORD_PAGES);
+        (void)hipFree(act);
+        rates = nullptr;
+        act = nullptr;
+      }
+      LSG_HIP(hipMalloc(&rates, (nw + 1 + WORD_PAGES) * 64 * sizeof(double)));
+      rates += 64 * WORD_PAGES;  // the slots' offsets; a uniform word has no rates
+      LSG_HIP(hipMalloc(&act, (nw + 1) * sizeof(uint64_t)));
+      ratesNw = nw;
+    }
+    return 0;
+  }
+  void release() {
+    for (WordStore &x : w) x.release();
+    init.release();
+    if (rates) (void)hipFree(rates - 64 * WORD_PAGES);
+    if (act) (void)hipFree(act);
+    if (st) (void)hipFree(st);
+    if (box) (void)hipFree(box);
+    box = nullptr;
+    boxSlots = 0;
+    rates = nullptr;
+    act = nullptr;
+    ratesNw = 0;
+    st = nullptr;
+  }
+};
+static WordWs g_words;
+static int g_domains = 0;  // level sets alive
+
 }  // namespace lsg
 
 using namespace lsg;
@@ -179,6 +279,10 @@ struct lsg_domain {
   Frame f{};
   int width = 1;
   Store cur, tmp;  // current band and the output buffer of the next op
+  // the band as a word band (lsg_words.hpp); which of the two forms hold it
+  WordStore words;
+  bool runsValid = true, wordsValid = false;
+  bool wordsOk = true;  // no run of defined points (only single points are defined)
   uint32_t hostN = 0;
   bool framed = false;
   std::vector<PdArray> pd;    // point data, insertion order
@@ -191,9 +295,23 @@ struct lsg_domain {
     }
     pd.clear();
   }
+  lsg_domain() { ++g_domains; }
+  lsg_domain(const lsg_domain &) = delete;
+  lsg_domain &operator=(const lsg_domain &) = delete;
+  // the run list was written: the word band is out of date
+  void runsChanged() {
+    runsValid = true;
+    wordsValid = false;
+  }
+  void wordsChanged() {
+    wordsValid = true;
+    runsValid = false;
+  }
   ~lsg_domain() {
+    if (--g_domains == 0) g_words.release();
     cur.release();
     tmp.release();
+    words.release();
     pdRelease();
     if (pdLen) (void)hipFree(pdLen);
   }
@@ -326,6 +444,18 @@ static int uploadRuns(lsg_domain *d, const std::vector<int32_t> &idx, const std:
     pos[i] = p;
     bits[p >> 6] |= 1ull << (p & 63);
   }
+  // a defined entry that is not followed by an entry at the next point is a
+  // run of defined points, which word bands do not hold
+  bool single = !(f.base && !isUndef(val[0]) && n > 0);
+  const uint32_t lastPoint = f.encode(f.ext[0] - 1, f.ext[1] - 1, f.ext[2] - 1);
+  for (size_t i = (size_t)f.base; i < n && single; ++i) {
+    if (isUndef(val[i]) || pos[i] == lastPoint) continue;
+    int32_t xr, yr, zr;
+    f.decode(pos[i], xr, yr, zr);
+    const uint32_t next = xr + 1 < f.ext[0] ? pos[i] + 1u : (((pos[i] >> 6) + 1u) << 6);
+    single = i + 1 < n && pos[i + 1] == next;
+  }
+  d->wordsOk = single;
   std::vector<uint32_t> pre(f.nwords + 1, 0);
   uint32_t acc = 0;
   for (int64_t w = 0; w <= f.nwords; ++w) {
@@ -343,11 +473,47 @@ static int uploadRuns(lsg_domain *d, const std::vector<int32_t> &idx, const std:
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
   d->hostN = nn;
   d->width = width;
+  d->runsChanged();
   return 0;
+}
+
+// Whether the operations on this level set run on word bands.
+static bool wordBands(const lsg_domain *d) {
+  return d->framed && d->wordsOk && d->pd.empty() && !singlePassBandOps() && d->f.nwords <= WORD_BAND_MAX_WORDS;
+}
+static int needWords(lsg_domain *d) {
+  if (d->wordsValid) return 0;
+  if (int e = d->words.ensure(d->f.nwords)) return e;
+  launchWordImport(g_ctx.s, d->cur.b, d->words.b, d->f);
+  d->wordsValid = true;
+  return 0;
+}
+// The run list of a band that only exists as a word band.
+static int needRuns(lsg_domain *d, bool mayAllocate = true) {
+  if (d->runsValid) return 0;
+  size_t cap = d->cur.b.cap;
+  for (int attempt = 0; attempt < 2; ++attempt) {
+    if (mayAllocate)
+      if (int e = ensureStores(d, cap ? cap : capFor(0))) return e;
+    if (!d->cur.b.val || d->cur.nwAlloc < d->f.nwords) return fail(-7, "level set has no run-list store");
+    launchWordExport(g_ctx.s, d->words.b, d->cur.b, d->f, d->g, g_ws->w.partials, g_ctx.stat + 7);
+    uint32_t n = 0;
+    LSG_HIP(hipMemcpyAsync(&n, g_ctx.stat + 7, sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
+    LSG_HIP(hipStreamSynchronize(g_ctx.s));
+    if (n <= d->cur.b.cap) {
+      d->hostN = n;
+      d->runsValid = true;
+      return 0;
+    }
+    if (!mayAllocate) break;
+    cap = capFor(n);
+  }
+  return fail(-40, "band capacity overflow");
 }
 
 static int downloadRuns(lsg_domain *d, std::vector<int32_t> &idx, std::vector<double> &val) {
   if (int e = ctxInit()) return e;
+  if (int e = needRuns(d)) return e;
   uint32_t n = 0;
   LSG_HIP(hipMemcpyAsync(&n, d->cur.b.n, sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
@@ -449,7 +615,11 @@ static void runsFromPoints(const lsg_domain *d, std::vector<int32_t> pidx, std::
 
 // ------------------------------------------------------------- ops ----
 
-static void swapCur(lsg_domain *d) { std::swap(d->cur, d->tmp); }
+static void swapCur(lsg_domain *d) {
+  std::swap(d->cur, d->tmp);
+  d->runsChanged();
+}
+static int maybeReframe(lsg_domain *d, bool force);
 
 // Event pairs around the evaluation kernel of star operations, taken from a
 // pool while an Advect with profiling on enqueues its step.
@@ -782,7 +952,8 @@ static int readOverflow(bool reset) {
 
 // Band statistics: defined count and absolute bounding box of in-frame entries.
 static int bandStats(lsg_domain *d, uint32_t &ndef, int32_t bbmin[3], int32_t bbmax[3], bool &any) {
-  launchBandStats(g_ctx.s, d->cur.b, d->f, g_ctx.stat, (int32_t *)(g_ctx.stat + 1));
+  if (d->runsValid) launchBandStats(g_ctx.s, d->cur.b, d->f, g_ctx.stat, (int32_t *)(g_ctx.stat + 1));
+  else launchWordStats(g_ctx.s, d->words.b, d->f, g_ctx.stat, (int32_t *)(g_ctx.stat + 1), nullptr, g_ctx.stat + 7);
   uint32_t h[7];
   LSG_HIP(hipMemcpyAsync(h, g_ctx.stat, 7 * sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
@@ -796,6 +967,93 @@ static int bandStats(lsg_domain *d, uint32_t &ndef, int32_t bbmin[3], int32_t bb
   return 0;
 }
 
+// A level set takes a result from a workspace band: the two are exchanged
+// when their sizes are close, else the result is copied (a small level set
+// does not keep a large store).
+static int takeWords(lsg_domain *d, WordStore &w) {
+  const int64_t a = d->words.nwAlloc, b = w.nwAlloc;
+  if (a >= d->f.nwords && a <= b + b / 2 && b <= a + a / 2) {
+    std::swap(w, d->words);
+  } else {
+    if (int e = d->words.ensure(d->f.nwords)) return e;
+    launchWordCopy(g_ctx.s, w.b, d->words.b, d->f);
+  }
+  d->wordsChanged();
+  return 0;
+}
+// Word band on another frame.
+static int reframeWords(lsg_domain *d, const Frame &f) {
+  if (int e = needWords(d)) return e;
+  if (int e = g_words.ensureOps(f.nwords)) return e;
+  launchWordReframe(g_ctx.s, d->words.b, d->f, d->g, g_words.w[0].b, f);
+  d->f = f;
+  return takeWords(d, g_words.w[0]);
+}
+// Whether a band with this bounding box comes too close to an open edge of
+// the frame.
+static bool nearFrameEdge(const lsg_domain *d, const int32_t bbmin[3], const int32_t bbmax[3]) {
+  for (int k = 0; k < d->D; ++k) {
+    if (d->g.bounded(k)) continue;
+    if (bbmin[k] - d->f.o[k] < REFRAME_SLACK || (d->f.o[k] + d->f.ext[k] - 1) - bbmax[k] < REFRAME_SLACK) return true;
+  }
+  return false;
+}
+// A sequence of operations on a level set's word band through the workspace
+// bands; the level set keeps its own until take().
+struct WordChain {
+  lsg_domain *d;
+  int at = -1;  // the current band: -1 the level set's store, else a workspace band
+  WordBufs store(int k) const { return k < 0 ? d->words.b : g_words.w[k].b; }
+  int other() const { return at == 0 ? 1 : 0; }
+  int begin() {
+    if (int e = needWords(d)) return e;
+    return g_words.ensureOps(d->f.nwords);
+  }
+  void star(int op, double a, double b = 0) {
+    WordOpArgs o;
+    o.a = a;
+    o.b = b;
+    launchWordStar(g_ctx.s, d->D, op, store(at), store(other()), d->f, d->g, o, g_words.st);
+    at = other();
+  }
+  void boolean(const WordBufs &B, int kind) {
+    launchWordBoolean(g_ctx.s, store(at), B, store(other()), d->f, kind, 0, 0);
+    at = other();
+  }
+  // Takes the result and moves the frame if the band has come close to its
+  // edge.  Returns 1, with the level set as before, when an Expand met a
+  // field that word bands do not hold: the caller uses the run list.
+  int take() {
+    launchWordStats(g_ctx.s, store(at), d->f, g_ctx.stat, (int32_t *)(g_ctx.stat + 1), g_words.st, g_ctx.stat + 7);
+    uint32_t h[8];
+    LSG_HIP(hipMemcpyAsync(h, g_ctx.stat, sizeof(h), hipMemcpyDeviceToHost, g_ctx.s));
+    LSG_HIP(hipStreamSynchronize(g_ctx.s));
+    if (h[7]) return wordConflict(d);
+    if (at >= 0)
+      if (int e = takeWords(d, g_words.w[at])) return e;
+    const int32_t *bb = (const int32_t *)(h + 1);
+    if (bb[0] > bb[3]) return 0;
+    int32_t mn[3], mx[3];
+    for (int k = 0; k < 3; ++k) {
+      mn[k] = bb[k] + d->f.o[k];
+      mx[k] = bb[3 + k] + d->f.o[k];
+    }
+    if (!nearFrameEdge(d, mn, mx)) return 0;
+    Frame f;
+    if (int e = makeFrame(d, mn, mx, f)) return e;
+    if (f.nwords <= WORD_BAND_MAX_WORDS) return reframeWords(d, f);
+    return maybeReframe(d, true);
+  }
+  // From here on the level set's operations run on its run list.
+  static int wordConflict(lsg_domain *d) {
+    LSG_HIP(hipMemsetAsync(&g_words.st->conflict, 0, sizeof(uint32_t), g_ctx.s));
+    d->wordsOk = false;
+    if (int e = needRuns(d)) return e;
+    d->runsChanged();
+    return 1;
+  }
+};
+
 // Move the frame when the band approached its edge in an infinite dimension.
 static int maybeReframe(lsg_domain *d, bool force) {
   uint32_t ndef;
@@ -803,13 +1061,12 @@ static int maybeReframe(lsg_domain *d, bool force) {
   bool any;
   if (int e = bandStats(d, ndef, bbmin, bbmax, any)) return e;
   if (!any) return 0;
-  bool need = force;
-  for (int k = 0; k < d->D; ++k) {
-    if (d->g.bounded(k)) continue;
-    if (bbmin[k] - d->f.o[k] < REFRAME_SLACK || (d->f.o[k] + d->f.ext[k] - 1) - bbmax[k] < REFRAME_SLACK)
-      need = true;
+  if (!force && !nearFrameEdge(d, bbmin, bbmax)) return 0;
+  if (!d->runsValid) {
+    Frame f;
+    if (int e = makeFrame(d, bbmin, bbmax, f)) return e;
+    if (f.nwords <= WORD_BAND_MAX_WORDS) return reframeWords(d, f);
   }
-  if (!need) return 0;
   std::vector<int32_t> idx;
   std::vector<double> val;
   if (int e = downloadRuns(d, idx, val)) return e;
@@ -848,7 +1105,13 @@ static int commonFrameAll(const std::vector<lsg_domain *> &ds) {
   }
   Frame f;
   if (int e = makeFrame(a, mn, mx, f)) return e;
+  bool words = f.nwords <= WORD_BAND_MAX_WORDS;
+  for (const lsg_domain *d : ds) words = words && wordBands(d);
   for (lsg_domain *d : ds) {
+    if (words) {
+      if (int e = reframeWords(d, f)) return e;
+      continue;
+    }
     std::vector<int32_t> idx;
     std::vector<double> val;
     if (int e = downloadRuns(d, idx, val)) return e;
@@ -902,6 +1165,14 @@ struct lsg_advect {
   StepGraph graphs[2];
   int nextGraph = 0;
   bool useGraphs = true;
+  // the captured step on word bands
+  struct WordGraph {
+    uint64_t key = 0;
+    hipGraphExec_t exec = nullptr;
+    int at = 0, width = 0, evUsed = 0, starUsed = 0;
+  } wordGraphs[2];
+  int nextWordGraph = 0;
+  lsg::WordStep *hostStep = nullptr;  // pinned
   double *hostMaxDt = nullptr;  // pinned, read by the step's first kernel
   double *devMaxDt = nullptr;
   lsg::DevScalars *hostSc = nullptr;  // pinned
@@ -931,6 +1202,10 @@ struct lsg_advect {
       if (g.exec) (void)hipGraphExecDestroy(g.exec);
       g = StepGraph{};
     }
+    for (auto &g : wordGraphs) {
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+      g = WordGraph{};
+    }
   }
   ~lsg_advect() {
     dropGraphs();
@@ -944,6 +1219,7 @@ struct lsg_advect {
     for (auto e : star2Pool) (void)hipEventDestroy(e);
     if (hostMaxDt) (void)hipHostFree(hostMaxDt);
     if (hostSc) (void)hipHostFree(hostSc);
+    if (hostStep) (void)hipHostFree(hostStep);
     if (hostStat) (void)hipHostFree(hostStat);
     if (mlpDev) (void)hipFree(mlpDev);
     for (void *p : {(void *)velIn, (void *)velOut, (void *)dlist, (void *)ndef, (void *)sllfIn, (void *)sllfOut})
@@ -1186,7 +1462,9 @@ static void copyDomainNoAlloc(lsg_domain *dst, const lsg_domain *src) {
   dst->f = src->f;
   dst->framed = src->framed;
   dst->width = src->width;
+  dst->wordsOk = src->wordsOk;
   launchCopyBand(g_ctx.s, src->cur.b, dst->cur.b, src->f);
+  dst->runsChanged();
   dst->hostN = src->hostN;
   (void)pdCopy(dst, src);
 }
@@ -1201,8 +1479,16 @@ static int copyDomain(lsg_domain *dst, const lsg_domain *src) {
   dst->f = src->f;
   dst->framed = src->framed;
   dst->width = src->width;
-  if (int e = ensureCur(dst, src->cur.nwAlloc, src->cur.b.cap)) return e;
-  launchCopyBand(g_ctx.s, src->cur.b, dst->cur.b, src->f);
+  dst->wordsOk = src->wordsOk;
+  if (src->runsValid) {
+    if (int e = ensureCur(dst, src->cur.nwAlloc, src->cur.b.cap)) return e;
+    launchCopyBand(g_ctx.s, src->cur.b, dst->cur.b, src->f);
+    dst->runsChanged();
+  } else {
+    if (int e = dst->words.ensure(src->f.nwords)) return e;
+    launchWordCopy(g_ctx.s, src->words.b, dst->words.b, src->f);
+    dst->wordsChanged();
+  }
   dst->hostN = src->hostN;
   return pdCopy(dst, src);
 }
@@ -1463,6 +1749,250 @@ static int runStep(lsg_advect *a, lsg_domain *d, double maxTimeStep, StepOut &ou
   return fail(-30, "band capacity overflow persists after retries");
 }
 
+// ------------------------------------------------- steps on word bands ---
+// One time step of one level set (Advect::advect, lsAdvect.hpp:817-830) on
+// word bands.  The level set's own store keeps the starting band; the
+// operations alternate between two workspace bands, and a Runge-Kutta step
+// keeps its expanded starting band in a third.  The level set then takes the
+// last band in exchange for its own.
+struct WordStepper {
+  lsg_advect *a;
+  lsg_domain *d;
+  int at = -1;  // current band: -1 the level set's store, else workspace band
+  int width;
+  bool begun = false;
+  WordBufs init;
+  WordBufs store(int k) const { return k < 0 ? d->words.b : g_words.w[k].b; }
+  int other() const { return at == 0 ? 1 : 0; }
+  void begin(WordOpArgs &o) {  // the step's first operation resets the scalars
+    if (!begun) o.begin = a->devMaxDt;
+    begun = true;
+  }
+  void launch(int op, const WordBufs &in, const WordBufs &out, const WordOpArgs &o) {
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    bool external = false;
+    if (op == W_EXPAND || op == W_REBUILD) takeEvents(a->profiling ? &a->starT : nullptr, e0, e1, external);
+    if (e0) (void)hipEventRecordWithFlags(e0, g_ctx.s, external ? hipEventRecordExternal : hipEventRecordDefault);
+    launchWordStar(g_ctx.s, d->D, op, in, out, d->f, d->g, o, g_words.st);
+    if (e1) (void)hipEventRecordWithFlags(e1, g_ctx.s, external ? hipEventRecordExternal : hipEventRecordDefault);
+  }
+  WordOpArgs expandArgs(int from, int cycle, int to) {
+    WordOpArgs o;
+    o.a = (from + cycle + 1) * 0.5;
+    o.b = to * 0.5;
+    o.count = a->profiling ? 1 : 0;
+    return o;
+  }
+  // `active`: the last cycle also writes the result's active points.
+  void expand(int to, bool active) {
+    const int from = width;
+    for (int c = 0; c < to - from; ++c) {
+      WordOpArgs o = expandArgs(from, c, to);
+      if (active && c == to - from - 1) o.act = g_words.act;
+      begin(o);
+      const int k = other();
+      launch(W_EXPAND, store(at), store(k), o);
+      at = k;
+    }
+    width = std::max(width, to);
+  }
+  // The starting band expanded: the last cycle writes the third workspace
+  // band, the ones before alternate with the free one of the other two.
+  void expandInit(int from, int to) {
+    init = d->words.b;
+    for (int c = 0; c < to - from; ++c) {
+      const WordBufs out = ((to - from - 1 - c) & 1) ? store(other()) : g_words.init.b;
+      launch(W_EXPAND, init, out, expandArgs(from, c, to));
+      init = out;
+    }
+  }
+  void stage(int k, const double *maxDt, bool isLast) {
+    const bool expands = width < prepareWidth(a->spatial);
+    expand(prepareWidth(a->spatial), true);
+    if (!expands) launchWordActive(g_ctx.s, store(at), d->f, g_words.act);
+    if (!begun) launchWordBegin(g_ctx.s, g_words.st, a->devMaxDt);
+    begun = true;
+    const int scheme = schemeIdOf(a->spatial);
+    RateParams rp = a->rp;
+    rp.hostVel = nullptr;
+    rp.hostSllf = nullptr;
+    rp.dissOut = nullptr;
+    rp.voidMarks = nullptr;
+    const WordBufs b = store(at);
+    if (scheme == S_LF) launchWordAlphas(g_ctx.s, d->D, b, d->f, d->g, rp, g_words.act, k, g_words.st);
+    hipEvent_t e0 = nullptr, e1 = nullptr;
+    if (a->profiling && a->evUsed + 2 <= (int)a->evPool.size()) {
+      e0 = a->evPool[a->evUsed];
+      e1 = a->evPool[a->evUsed + 1];
+      a->evUsed += 2;
+    }
+    double *box = scheme == S_LLF && boxAlphasShared(d->g, d->f, velOf(rp)) ? g_words.box : nullptr;
+    launchWordRates(g_ctx.s, d->D, b, d->f, d->g, rp, g_words.act, g_words.rates, box, k, a->profiling ? 1 : 0,
+                    g_words.st, e0, e1, a->capturing);
+    const bool sllf = a->spatial == 9;
+    WordOpArgs o;
+    o.a = sllf ? 1.5 : 1.0;  // doRebuild's cutoff
+    o.stage = k;
+    o.useAlphas = scheme == S_LF || scheme == S_LLLF || scheme == S_LLF || scheme == S_LLFA || scheme == S_SLLF;
+    o.cfl = a->cfl;
+    o.maxDt = maxDt;
+    o.rates = g_words.rates;
+    o.inAct = g_words.act;
+    if (isLast) o.slack = REFRAME_SLACK;
+    const int n = other();
+    launch(W_UPD_REBUILD, b, store(n), o);
+    at = n;
+    width = sllf ? 3 : 2;
+  }
+  void combine(double wTarget, double wSource, bool first, int initWidth, bool isLast) {
+    const int steps = a->temporal == 1 ? 2 : 3;
+    const int ew = (int)std::ceil(2.0 * steps * a->cfl + 1);
+    expand(ew, false);
+    if (first) expandInit(initWidth, ew);
+    int n = other();
+    launchWordBoolean(g_ctx.s, store(at), init, store(n), d->f, B_COMBINE, wTarget, wSource);
+    at = n;
+    for (int op : {W_PRUNE_RSZ, W_PRUNE}) {
+      n = other();
+      launch(op, store(at), store(n), WordOpArgs{});
+      at = n;
+    }
+    const bool sllf = a->spatial == 9;
+    WordOpArgs o;
+    o.a = sllf ? 1.5 : 1.0;
+    o.count = a->profiling ? 1 : 0;
+    if (isLast) o.slack = REFRAME_SLACK;
+    n = other();
+    launch(W_REBUILD, store(at), store(n), o);
+    at = n;
+    width = sllf ? 3 : 2;
+  }
+};
+
+// Returns the workspace band that holds the result.
+static int enqueueWordStep(lsg_advect *a, lsg_domain *d) {
+  const WordStep *st = g_words.st;
+  a->evUsed = 0;
+  a->starT = StarTiming{a->starPool.data(), (int)a->starPool.size(), 0, a->capturing};
+  WordStepper s{a, d};
+  s.width = d->width;
+  const int initWidth = d->width;
+  const bool fe = a->temporal == 0, rk2 = a->temporal == 1;
+  s.stage(0, &st->maxTimeStep, fe);
+  if (!fe) {
+    s.stage(1, &st->dt[0], false);
+    s.combine(rk2 ? 0.5 : 0.75, rk2 ? 0.5 : 0.25, true, initWidth, rk2);
+    if (!rk2) {
+      s.stage(2, &st->dt[0], false);
+      s.combine(1.0 / 3.0, 2.0 / 3.0, false, initWidth, true);
+    }
+  }
+  d->width = s.width;
+  return s.at;
+}
+
+// Returns 1, with the level set as before, when an Expand met a field that
+// word bands do not hold: the caller advects the run list.
+static int runWordStep(lsg_advect *a, lsg_domain *d, double maxTimeStep, StepOut &out) {
+  if (int e = needWords(d)) return e;
+  if (int e = g_words.ensureStep(d->f.nwords, a->temporal != 0)) return e;
+  if (schemeIdOf(a->spatial) == S_LLF && boxAlphasShared(d->g, d->f, velOf(a->rp)))
+    if (int e = g_words.ensureBox(d->f.nwords, d->D)) return e;
+  if (!a->hostStep) LSG_HIP(hipHostMalloc((void **)&a->hostStep, sizeof(WordStep), hipHostMallocDefault));
+  *a->hostMaxDt = maxTimeStep;
+  const int widthBefore = d->width;
+  int at = 0;
+  if (a->useGraphs) {
+    uint64_t key = 1469598103934665603ull;
+    auto add = [&](const void *p, size_t n) { key = fnv(key, p, n); };
+    add(&d->words.b, sizeof(WordBufs));
+    for (const WordStore *w : {&g_words.w[0], &g_words.w[1], &g_words.init}) add(&w->b, sizeof(WordBufs));
+    add(&g_words.rates, sizeof(double *));
+    add(&g_words.act, sizeof(uint64_t *));
+    add(&g_words.box, sizeof(double *));
+    add(&g_words.st, sizeof(WordStep *));
+    add(&d->f, sizeof(Frame));
+    add(&d->g, sizeof(GridInfo));
+    add(&d->width, sizeof(int));
+    add(&a->rp, sizeof(RateParams));
+    add(&a->temporal, sizeof(int));
+    add(&a->cfl, sizeof(double));
+    add(&a->profiling, sizeof(bool));
+    lsg_advect::WordGraph *hit = nullptr;
+    for (auto &c : a->wordGraphs)
+      if (c.exec && c.key == key) hit = &c;
+    lsg_advect::WordGraph &g = hit ? *hit : a->wordGraphs[a->nextWordGraph];
+    if (hit) {
+      at = g.at;
+      d->width = g.width;
+      a->evUsed = g.evUsed;
+      a->starT.used = g.starUsed;
+    } else {
+      a->nextWordGraph ^= 1;
+      if (g.exec) (void)hipGraphExecDestroy(g.exec);
+      g = lsg_advect::WordGraph{};
+      hipGraph_t graph = nullptr;
+      bool ok = hipStreamBeginCapture(g_ctx.s, hipStreamCaptureModeThreadLocal) == hipSuccess;
+      if (ok) {
+        a->capturing = true;
+        at = enqueueWordStep(a, d);
+        a->capturing = false;
+        ok = hipStreamEndCapture(g_ctx.s, &graph) == hipSuccess && graph;
+      }
+      if (ok) ok = hipGraphInstantiate(&g.exec, graph, nullptr, nullptr, 0) == hipSuccess;
+      if (graph) (void)hipGraphDestroy(graph);
+      if (!ok) {
+        // capture unsupported here: direct launches for good
+        (void)hipGetLastError();
+        a->useGraphs = false;
+        a->dropGraphs();
+        d->width = widthBefore;
+        return fail(-31, "HIP graph capture failed; retry the call (direct launches are used from now on)");
+      }
+      g.key = key;
+      g.at = at;
+      g.width = d->width;
+      g.evUsed = a->evUsed;
+      g.starUsed = a->starT.used;
+    }
+    LSG_HIP(hipGraphLaunch(g.exec, g_ctx.s));
+  } else {
+    at = enqueueWordStep(a, d);
+  }
+  const size_t bytes = a->profiling ? sizeof(WordStep) : offsetof(WordStep, maxAbs);
+  LSG_HIP(hipMemcpyAsync(a->hostStep, g_words.st, bytes, hipMemcpyDeviceToHost, g_ctx.s));
+  LSG_HIP(hipStreamSynchronize(g_ctx.s));
+  const WordStep &h = *a->hostStep;
+  if (h.conflict) {
+    d->width = widthBefore;
+    return WordChain::wordConflict(d);
+  }
+  if (int e = takeWords(d, g_words.w[at])) return e;
+  // the returned time (lsAdvectIntegrationSchemes.hpp:58,107,167)
+  out.dt1 = h.dt[0];
+  if (a->temporal == 1) out.stepTime = 0.5 * h.dt[0] + 0.5 * h.dt[1];
+  else if (a->temporal == 2) out.stepTime = (h.dt[0] + h.dt[1] + 4.0 * h.dt[2]) / 6.0;
+  else out.stepTime = h.dt[0];
+  out.active = 0;
+  for (int k = 0; k < STEP_STAGES; ++k)
+    for (int i = 0; i < STEP_SLOTS; ++i) out.active += h.active[k][i];
+  if (a->profiling) {
+    auto take = [](std::vector<hipEvent_t> &ev, int used, double &ms, int64_t &n) {
+      for (int k = 0; k + 1 < used; k += 2) {
+        float t = 0;
+        if (hipEventElapsedTime(&t, ev[k], ev[k + 1]) == hipSuccess) {
+          ms += t;
+          n += 1;
+        }
+      }
+    };
+    take(a->evPool, a->evUsed, a->rateMs, a->rateLaunches);
+    take(a->starPool, a->starT.used, a->starMs, a->starLaunches);
+  }
+  if (h.reframe) return maybeReframe(d, true);
+  return 0;
+}
+
 // ---------------------------------------------------- several level sets ---
 // Advect with level sets below the advected top (lsAdvect.hpp:435-612,
 // 686-813; lsAdvectIntegrationSchemes.hpp:46-168).  All level sets share
@@ -1590,6 +2120,10 @@ static int runStepMM(lsg_advect *a, double maxTimeStep, StepOut &out) {
   const size_t L = a->levelSets.size();
   for (int attempt = 0; attempt < 6; ++attempt) {
     if (int e = commonFrameAll(a->levelSets)) return e;
+    for (lsg_domain *d : a->levelSets) {
+      if (int e = needRuns(d)) return e;
+      d->runsChanged();
+    }
     size_t cap = top->cur.b.cap;
     for (lsg_domain *d : a->levelSets) cap = std::max(cap, d->cur.b.cap);
     for (lsg_domain *d : a->levelSets)
@@ -1686,13 +2220,26 @@ static int advectApply(lsg_advect *a) {
     const char *e = getenv("LSG_LEARNED_WAVE");
     a->rp.learnedWave = (e && e[0] == '0') ? 0 : 1;
   }
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
-  if (int e = ensureRates(a, d->cur.b.cap)) return e;
-  if (a->temporal != 0) {
-    if (!a->init) a->init = new lsg_domain();
-    if (int e = copyDomain(a->init, d)) return e;
-    if (int e = ensureStores(a->init, d->cur.b.cap)) return e;
-  }
+  // steps on word bands: one level set with device-evaluated velocities and
+  // nothing to do between the stages; the others read run lists
+  bool words = !multi && wordBands(d) && !a->hostScalar && !a->hostVector && !a->saveVelocities && !a->ignoreVoids &&
+               !(a->velUpdate && a->temporal != 0) && a->spatial != 12;
+  auto prepareRuns = [&]() -> int {
+    for (lsg_domain *l : a->levelSets) {
+      if (int e = needRuns(l)) return e;
+      l->runsChanged();
+    }
+    if (int e = ensureStores(d, d->cur.b.cap)) return e;
+    if (int e = ensureRates(a, d->cur.b.cap)) return e;
+    if (a->temporal != 0) {
+      if (!a->init) a->init = new lsg_domain();
+      if (int e = copyDomain(a->init, d)) return e;
+      if (int e = ensureStores(a->init, d->cur.b.cap)) return e;
+    }
+    return 0;
+  };
+  if (!words)
+    if (int e = prepareRuns()) return e;
   if (!a->hostMaxDt) {
     LSG_HIP(hipHostMalloc((void **)&a->hostMaxDt, sizeof(double), hipHostMallocMapped | hipHostMallocCoherent));
     LSG_HIP(hipHostGetDevicePointer((void **)&a->devMaxDt, a->hostMaxDt, 0));
@@ -1710,7 +2257,15 @@ static int advectApply(lsg_advect *a) {
   if (const char *ng = getenv("LSG_NO_GRAPH")) a->useGraphs = (ng[0] == '0');
   a->pointUpdates = 0;
   StepOut so{};
-  auto step = [&](double maxT) { return multi ? runStepMM(a, maxT, so) : runStep(a, d, maxT, so); };
+  auto step = [&](double maxT) -> int {
+    if (words) {
+      const int r = runWordStep(a, d, maxT, so);
+      if (r != 1) return r;
+      words = false;
+      if (int e = prepareRuns()) return e;
+    }
+    return multi ? runStepMM(a, maxT, so) : runStep(a, d, maxT, so);
+  };
   if (a->advectionTime == 0.) {
     if (int e = step(std::numeric_limits<double>::max())) return e;
     a->advectedTime = so.stepTime;
@@ -1731,7 +2286,13 @@ static int advectApply(lsg_advect *a) {
   }
   a->currentTimeStep = so.dt1;
   if (a->temporal == 0) a->currentTimeStep = so.stepTime;
-  if (a->profiling) {
+  if (a->profiling && words) {
+    a->rateBytes = a->starBytes = 0;
+    for (int i = 0; i < STEP_SLOTS; ++i) {
+      a->rateBytes += a->hostStep->rateBytes[i];
+      a->starBytes += a->hostStep->starBytes[i];
+    }
+  } else if (a->profiling) {
     a->rateBytes = a->hostSc->rateBytes;
     a->starBytes = a->hostSc->starBytes;
     a->star2Bytes = a->hostSc->star2Bytes;
@@ -1874,6 +2435,8 @@ static int ensureBatchWs(size_t cap, int64_t nw) {
 static int batchAssemble(lsg_batch *b) {
   const size_t S = b->doms.size();
   b->freeDevice();
+  for (lsg_domain *d : b->doms)
+    if (int e = needRuns(d)) return e;
   std::vector<uint32_t> nEnt(S);
   b->segsH.resize(S);
   int64_t W = 0;
@@ -1983,6 +2546,7 @@ static int batchWriteBack(lsg_batch *b) {
     LSG_HIP(hipMemcpyAsync(d->cur.b.val, o.val + e0, n * sizeof(double), hipMemcpyDeviceToDevice, g_ctx.s));
     LSG_HIP(hipMemcpyAsync(d->cur.b.pos, o.pos + e0, n * sizeof(uint32_t), hipMemcpyDeviceToDevice, g_ctx.s));
     kSetScalar32<<<1, 1, 0, g_ctx.s>>>(d->cur.b.n, n);
+    d->runsChanged();
     d->hostN = n;
     d->width = b->width;
   }
@@ -2307,6 +2871,7 @@ int lsg_domain_set_runs(lsg_domain *d, int64_t n, const int32_t *idx, const doub
 }
 
 int lsg_domain_num_runs(lsg_domain *d, int64_t *n) {
+  if (int e = needRuns(d)) return e;
   uint32_t h = 0;
   LSG_HIP(hipMemcpyAsync(&h, d->cur.b.n, sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
@@ -2566,6 +3131,8 @@ int lsg_domain_deserialize(lsg_domain *d, const uint8_t *buf, int64_t size) {
   d->width = t->width;
   if (int e = ensureCur(d, t->cur.nwAlloc, t->cur.b.cap)) return e;
   launchCopyBand(g_ctx.s, t->cur.b, d->cur.b, t->f);
+  d->wordsOk = t->wordsOk;
+  d->runsChanged();
   d->hostN = t->hostN;
   if (hasPointData == 1) {
     pdClear(d);
@@ -2596,6 +3163,7 @@ struct SurfBuf {
   }
 };
 static int surfaceOf(lsg_domain *d, SurfBuf &s) {
+  if (int e = needRuns(d)) return e;
   if (int e = ensureStores(d, d->cur.b.cap)) return e;
   uint32_t ne = 0;
   LSG_HIP(hipMemcpyAsync(&ne, d->cur.b.n, sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
@@ -2651,7 +3219,10 @@ static int afterOp(lsg_domain *d);
 static int judgeInput(lsg_domain *d, int minWidth, std::unique_ptr<lsg_domain> &copy, lsg_domain *&use) {
   use = d;
   if (d->width >= minWidth) return 0;
+  // on the run list: a word band made for one expansion of a copy costs more
+  // (its store, the import and the export) than the cycles it saves
   copy.reset(new lsg_domain());
+  if (int e = needRuns(d)) return e;
   if (int e = copyDomain(copy.get(), d)) return e;
   if (int e = ensureStores(copy.get(), copy->cur.b.cap)) return e;
   doExpand(copy.get(), minWidth);
@@ -2729,6 +3300,7 @@ int lsg_compare_volume(lsg_domain *target0, lsg_domain *sample0, uint64_t *cells
   int64_t bmin[3], bmax[3];
   bool any = false;
   for (lsg_domain *d : {A, B}) {
+    if (int e = needRuns(d)) return e;
     launchBandStats(g_ctx.s, d->cur.b, d->f, g_ctx.stat, (int32_t *)(g_ctx.stat + 1), 1u);
     int32_t h[7];
     LSG_HIP(hipMemcpyAsync(h, g_ctx.stat, 7 * sizeof(int32_t), hipMemcpyDeviceToHost, g_ctx.s));
@@ -2779,6 +3351,7 @@ int lsg_compare_volume(lsg_domain *target0, lsg_domain *sample0, uint64_t *cells
 int lsg_mark_void_points(lsg_domain *d) {
   if (int e = ctxInit()) return e;
   if (!d->framed) return fail(-7, "MarkVoidPoints: level set has no data");
+  if (int e = needRuns(d)) return e;
   if (int e = ensureStores(d, d->cur.b.cap)) return e;
   RateParams rp{};
   if (int e = markVoids(d, rp)) return e;
@@ -2867,11 +3440,30 @@ static int afterOp(lsg_domain *d) {
   return maybeReframe(d, false);
 }
 
-int lsg_expand(lsg_domain *d, int width) {
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
+// Expand, Reduce, Prune, rebuildLS and the booleans of a level set: on its
+// word band, or on the run list (point data to carry, the single-pass
+// kernels, a frame too large, a run of defined points).
+static int opOnRuns(lsg_domain *d) {
+  if (int e = needRuns(d)) return e;
+  return ensureStores(d, d->cur.b.cap);
+}
+static int expandDomain(lsg_domain *d, int width) {
+  if (wordBands(d)) {
+    WordChain c{d};
+    if (int e = c.begin()) return e;
+    for (int w = d->width; w < width; ++w) c.star(W_EXPAND, (w + 1) * 0.5, width * 0.5);
+    const int r = c.take();
+    if (r != 1) {
+      if (r == 0) d->width = std::max(d->width, width);
+      return r;
+    }
+  }
+  if (int e = opOnRuns(d)) return e;
   doExpand(d, width);
   return afterOp(d);
 }
+
+int lsg_expand(lsg_domain *d, int width) { return expandDomain(d, width); }
 
 // Expand without allocating: the cycles of lsg_expand (doExpand) as
 // single-pass star kernels whose flags, statistics and tile status words
@@ -2881,6 +3473,7 @@ int lsg_expand(lsg_domain *d, int width) {
 // the last complete cycle (the width says which).
 int lsg_expand_noalloc(lsg_domain *d, int width) {
   if (!g_ctx.init || !d->framed) return fail(-7, "lsg_expand_noalloc: level set has no data");
+  if (int e = needRuns(d, false)) return e;
   int cur = -1;
   LSG_HIP(hipGetDevice(&cur));
   if (cur != g_ctx.dev) return fail(-50, "lsg_expand_noalloc: the library runs on device " + std::to_string(g_ctx.dev));
@@ -2945,17 +3538,39 @@ int lsg_expand_noalloc(lsg_domain *d, int width) {
   return 0;
 }
 int lsg_reduce(lsg_domain *d, int width) {
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
+  if (wordBands(d)) {
+    WordChain c{d};
+    if (int e = c.begin()) return e;
+    if (width < d->width) c.star(W_REDUCE, width * 0.5);
+    const int r = c.take();
+    if (r == 0) d->width = std::min(d->width, width);
+    return r;
+  }
+  if (int e = opOnRuns(d)) return e;
   doReduce(d, width);
   return afterOp(d);
 }
 int lsg_prune(lsg_domain *d, int rsz) {
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
+  if (wordBands(d)) {
+    WordChain c{d};
+    if (int e = c.begin()) return e;
+    c.star(rsz ? W_PRUNE_RSZ : W_PRUNE, 0);
+    d->width = 2;
+    return c.take();
+  }
+  if (int e = opOnRuns(d)) return e;
   doPrune(d, rsz != 0);
   return afterOp(d);
 }
 int lsg_rebuild(lsg_domain *d) {
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
+  if (wordBands(d)) {
+    WordChain c{d};
+    if (int e = c.begin()) return e;
+    c.star(W_REBUILD, 1.0);
+    d->width = 2;
+    return c.take();
+  }
+  if (int e = opOnRuns(d)) return e;
   doRebuild(d);
   return afterOp(d);
 }
@@ -2963,12 +3578,30 @@ int lsg_boolean(lsg_domain *a, const lsg_domain *b, int op) {
   if (op == 3) {  // INVERT: b is not used (lsBooleanOperation.hpp:214-247)
     if (int e = ctxInit()) return e;
     if (!a->framed) return fail(-7, "BooleanOperation: level set has no data");
-    launchNegate(g_ctx.s, a->cur.b);
+    if (a->runsValid) {
+      launchNegate(g_ctx.s, a->cur.b);
+      a->runsChanged();
+    } else {
+      launchWordNegate(g_ctx.s, a->words.b, a->f);
+    }
     LSG_HIP(hipStreamSynchronize(g_ctx.s));
     return 0;
   }
   if (op < 0 || op > 2) return fail(-1, "unsupported boolean operation");
-  if (int e = commonFrame(a, const_cast<lsg_domain *>(b))) return e;
+  lsg_domain *bm = const_cast<lsg_domain *>(b);
+  if (int e = commonFrame(a, bm)) return e;
+  if (wordBands(a) && wordBands(b)) {  // the boolean, then pruning (doBoolean)
+    if (int e = needWords(bm)) return e;
+    WordChain c{a};
+    if (int e = c.begin()) return e;
+    c.boolean(b->words.b, op);
+    c.star(W_PRUNE_RSZ, 0);
+    c.star(W_PRUNE, 0);
+    a->width = 2;
+    return c.take();
+  }
+  if (int e = needRuns(a)) return e;
+  if (int e = needRuns(bm)) return e;
   if (int e = ensureStores(a, std::max(a->cur.b.cap, b->cur.b.cap))) return e;
   doBoolean(a, b, op, 0, 0);
   return afterOp(a);
@@ -3121,10 +3754,7 @@ int lsg_advect_prepare_ls(lsg_advect *a) {
   if (a->levelSets.empty()) return fail(-1, "No level sets passed to Advect.");
   int w = prepareWidth(a->spatial);
   if (w < 0) return fail(-1, "Advect: Discretization scheme not found.");
-  lsg_domain *d = a->levelSets.back();
-  if (int e = ensureStores(d, d->cur.b.cap)) return e;
-  doExpand(d, w);
-  return afterOp(d);
+  return expandDomain(a->levelSets.back(), w);
 }
 int lsg_advect_apply(lsg_advect *a) {
   if (g_inVelocityUpdate) return fail(-1, "Advect::apply called from a velocity update callback");
@@ -3158,6 +3788,10 @@ int lsg_advect_set_profiling(lsg_advect *a, int on) {
   LSG_HIP(hipMemcpy(&g_ctx.sc->rateBytes, &z, sizeof(double), hipMemcpyHostToDevice));
   LSG_HIP(hipMemcpy(&g_ctx.sc->starBytes, &z, sizeof(double), hipMemcpyHostToDevice));
   LSG_HIP(hipMemcpy(&g_ctx.sc->star2Bytes, &z, sizeof(double), hipMemcpyHostToDevice));
+  if (g_words.st) {
+    LSG_HIP(hipStreamSynchronize(g_ctx.s));
+    LSG_HIP(hipMemset(g_words.st, 0, sizeof(WordStep)));
+  }
   a->profiling = on != 0;
   a->rateMs = 0;
   a->rateLaunches = 0;

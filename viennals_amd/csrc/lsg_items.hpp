@@ -281,8 +281,8 @@ LSG_HD inline double updateRateMM(double c, double dt, const double *list, int &
 // along each unbounded axis, where the mapping is the identity.  -1
 // otherwise.  A located point is then exactly that index with inside =
 // true, and a boundary costs a few selects instead of locate() and map().
-template <int D> LSG_HD inline int64_t axisStride(const BandView &b, int d);
-template <int D, int R> LSG_HD inline int64_t mappedLin(const BandView &b, const int32_t c[3], int64_t off[][2 * R + 1]) {
+template <int D, class V> LSG_HD inline int64_t axisStride(const V &b, int d);
+template <int D, int R, class V> LSG_HD inline int64_t mappedLin(const V &b, const int32_t c[3], int64_t off[][2 * R + 1]) {
   bool ok = true;
   LSG_UNROLL
   for (int d = 0; d < D; ++d) {
@@ -320,13 +320,13 @@ LSG_HD inline BandView::Loc locAt(int64_t lin) {
   l.inside = true;
   return l;
 }
-template <int D> LSG_HD inline int64_t axisStride(const BandView &b, int d) {
+template <int D, class V> LSG_HD inline int64_t axisStride(const V &b, int d) {
   return d == 0 ? 1 : (d == 1 ? (int64_t)b.f.rowBits() : (int64_t)b.f.ext[1] * b.f.rowBits());
 }
 
 // Centre value and the 2D star neighbours (boundary mapped) of point c:
 // nb[d] = +e_d, nb[D + d] = -e_d.  All 2D + 1 lookups are issued together.
-template <int D> LSG_HD inline void starLocs(const BandView &b, const int32_t c[3], BandView::Loc *l) {
+template <int D, class V> LSG_HD inline void starLocs(const V &b, const int32_t c[3], BandView::Loc *l) {
   int64_t off[3][3];
   const int64_t lin = mappedLin<D, 1>(b, c, off);
   if (lin >= 0) {
@@ -349,11 +349,11 @@ template <int D> LSG_HD inline void starLocs(const BandView &b, const int32_t c[
     l[D + d] = b.locate(q[0], q[1], q[2]);
   }
 }
-template <int D> LSG_HD inline void gatherStar(const BandView &b, const int32_t c[3], double &center, double *nb) {
+template <int D, class V> LSG_HD inline void gatherStar(const V &b, const int32_t c[3], double &center, double *nb) {
   BandView::Loc l[2 * D + 1];
   starLocs<D>(b, c, l);
   double v[2 * D + 1];
-  b.values<2 * D + 1>(l, v);
+  b.template values<2 * D + 1>(l, v);
   LSG_UNROLL
   for (int k = 0; k < 2 * D; ++k) nb[k] = v[k];
   center = v[2 * D];
@@ -361,7 +361,7 @@ template <int D> LSG_HD inline void gatherStar(const BandView &b, const int32_t 
 // Values along every axis of point c up to distance R (boundary mapped):
 // st[d][R + k] = phi(c + k e_d) for 0 < |k| <= R; st[d][R] is left to the
 // caller (the centre value).  All 2 D R lookups are issued together.
-template <int D, int R> LSG_HD inline void gatherAxes(const BandView &b, const int32_t c[3], double st[][2 * R + 1]) {
+template <int D, int R, class V> LSG_HD inline void gatherAxes(const V &b, const int32_t c[3], double st[][2 * R + 1]) {
   BandView::Loc l[2 * D * R];
   int64_t off[3][2 * R + 1];
   const int64_t lin = mappedLin<D, R>(b, c, off);
@@ -389,7 +389,7 @@ template <int D, int R> LSG_HD inline void gatherAxes(const BandView &b, const i
   }
   }
   double v[2 * D * R];
-  b.values<2 * D * R>(l, v);
+  b.template values<2 * D * R>(l, v);
   LSG_UNROLL
   for (int d = 0; d < D; ++d) {
     LSG_UNROLL
@@ -539,7 +539,7 @@ LSG_HD inline double expandTwice(const BandView &b, const int32_t c[3], double l
         }
     }
     double v[N1];
-    b.values<N1>(l, v);
+    b.template values<N1>(l, v);
     double mn = POS, mx = NEG;
     LSG_UNROLL
     for (int k = 0; k < 2 * D; ++k) minMaxAcc(v[1 + k], mn, mx);
@@ -586,7 +586,7 @@ LSG_HD inline double expandTwice(const BandView &b, const int32_t c[3], double l
           }
         }
     double w[4 * D];
-    b.values<4 * D>(l, w);
+    b.template values<4 * D>(l, w);
     LSG_UNROLL
     for (int a = 0; a < D; ++a)
       LSG_UNROLL
@@ -875,7 +875,7 @@ struct Vel {
       for (int i = 0; i < 3; ++i) s += fabs(n[i]);
       return b + aPos * s;
     }
-    double c = n[dir];
+    double c = dir == 0 ? n[0] : (dir == 1 ? n[1] : n[2]);  // no indexed register access
     double a = (c > 0) ? aPos : aNeg;
     double ac = fabs(c);
     double m = 1.0;
@@ -992,7 +992,7 @@ LSG_HD inline void upwindDiffs(const double *st, double gridDelta, int order, do
 
 // Axis values at offsets -2..2 for the first/second-order schemes (the
 // second-order layer only when order == 2).
-template <int D> LSG_HD inline void gatherUpwind(const BandView &b, const int32_t c[3], int order, double st[][5]) {
+template <int D, class V> LSG_HD inline void gatherUpwind(const V &b, const int32_t c[3], int order, double st[][5]) {
   if (order == 2) {
     gatherAxes<D, 2>(b, c, st);
   } else {
@@ -1157,8 +1157,8 @@ struct RateOut {
 };
 
 // EngquistOsher::operator() (lsEngquistOsher.hpp:42-162)
-template <int D>
-LSG_HD inline RateOut schemeEO(const BandView &b, const int32_t c[3], double phi0, int order, bool calcNormals,
+template <int D, class V>
+LSG_HD inline RateOut schemeEO(const V &b, const int32_t c[3], double phi0, int order, bool calcNormals,
                                const Vel &vel) {
   double gradPos[D], gradNeg[D];
   double gradPosTotal = 0, gradNegTotal = 0;
@@ -1279,8 +1279,8 @@ LSG_HD inline void weno5LearnedAxes(double sts[][7], double dx, const float *P, 
 // Learned weno5 in two phases can keep the axis values of the first in
 // `stc` (element q of the D x 7 values at stc[q * stcStride]): the second
 // phase then reads them there instead of gathering them again.
-template <int D, int ORDER, bool LEARNED = false>
-LSG_HD inline RateOut schemeWENO(const BandView &b, const int32_t c[3], double phi0, bool calcNormals, const Vel &vel,
+template <int D, int ORDER, bool LEARNED = false, class V>
+LSG_HD inline RateOut schemeWENO(const V &b, const int32_t c[3], double phi0, bool calcNormals, const Vel &vel,
                                  const float *mlp = nullptr, float *io = nullptr, int phase = 0,
                                  const double *stc = nullptr, int stcStride = 0) {
   constexpr int r = (ORDER + 1) / 2;
@@ -1345,8 +1345,8 @@ LSG_HD inline RateOut schemeWENO(const BandView &b, const int32_t c[3], double p
 }
 
 // LaxFriedrichs::operator() (lsLaxFriedrichs.hpp:46-158)
-template <int D>
-LSG_HD inline RateOut schemeLF(const BandView &b, const int32_t c[3], double phi0, int order, bool calcNormals,
+template <int D, class V>
+LSG_HD inline RateOut schemeLF(const V &b, const int32_t c[3], double phi0, int order, bool calcNormals,
                                const Vel &vel, double alphaFactor, const double *alphas) {
   double gradPos[D], gradNeg[D];
   double grad = 0., dissipation = 0.;
@@ -1384,8 +1384,8 @@ LSG_HD inline RateOut schemeLF(const BandView &b, const int32_t c[3], double phi
 }
 
 // LocalLocalLaxFriedrichs::operator() (lsLocalLocalLaxFriedrichs.hpp:42-165)
-template <int D>
-LSG_HD inline RateOut schemeLLLF(const BandView &b, const int32_t c[3], double phi0, int order, const Vel &vel,
+template <int D, class V>
+LSG_HD inline RateOut schemeLLLF(const V &b, const int32_t c[3], double phi0, int order, const Vel &vel,
                                  double alphaFactor, double *alphaAcc) {
   double gradPos[D], gradNeg[D];
   double grad = 0., dissipation = 0.;
@@ -1429,8 +1429,8 @@ LSG_HD inline RateOut schemeLLLF(const BandView &b, const int32_t c[3], double p
 // velocity field's analytical alphas (the built-in functor's are constant
 // per direction, so the 3^D box of normals does not enter), no dissipation
 // factor.
-template <int D>
-LSG_HD inline RateOut schemeLLFA(const BandView &b, const int32_t c[3], double phi0, const Vel &vel, double *alphaAcc) {
+template <int D, class V>
+LSG_HD inline RateOut schemeLLFA(const V &b, const int32_t c[3], double phi0, const Vel &vel, double *alphaAcc) {
   double gradPos[D], gradNeg[D];
   double grad = 0., dissipation = 0.;
   double n[3] = {0, 0, 0};
@@ -1501,7 +1501,7 @@ LSG_HD inline void llfaBoxDiffs(const BandView &b, const int32_t c[3], int q, do
     l[D + dir] = b.locate(pn[0], pn[1], pn[2]);
   }
   double v[2 * D + 1];
-  b.values<2 * D + 1>(l, v);
+  b.template values<2 * D + 1>(l, v);
   out[0] = out[1] = out[2] = 0.;
   LSG_UNROLL
   for (int dir = 0; dir < D; ++dir) {
@@ -1518,8 +1518,8 @@ LSG_HD inline void llfaBoxDiffs(const BandView &b, const int32_t c[3], int q, do
 // and D + dir its neighbours along dir (+, -).  With lin >= 0 (mappedLin
 // with R = 2) every point is a frame bit at its mapped offset; otherwise
 // each is located.
-template <int D>
-LSG_HD inline void llfBoxLocs(const BandView &b, const int32_t c[3], int q, int64_t lin, const int64_t off[][5],
+template <int D, class V>
+LSG_HD inline void llfBoxLocs(const V &b, const int32_t c[3], int q, int64_t lin, const int64_t off[][5],
                               BandView::Loc *l) {
   const int ni[3] = {q % 3 - 1, (q / 3) % 3 - 1, q / 9 - 1};
   if (lin >= 0) {
@@ -1569,17 +1569,17 @@ template <int D> LSG_HD inline void llfBoxNormalFrom(const double *bv, double dx
   LSG_UNROLL
   for (int dir = 0; dir < D; ++dir) normal[dir] *= nm;
 }
-template <int D> LSG_HD inline void llfBoxNormal(const BandView &b, const int32_t c[3], int q, double normal[3]) {
+template <int D, class V> LSG_HD inline void llfBoxNormal(const V &b, const int32_t c[3], int q, double normal[3]) {
   BandView::Loc l[2 * D + 1];
   llfBoxLocs<D>(b, c, q, -1, nullptr, l);
   double bv[2 * D + 1];
-  b.values<2 * D + 1>(l, bv);
+  b.template values<2 * D + 1>(l, bv);
   llfBoxNormalFrom<D>(bv, b.g.dx, normal);
 }
 
 // LocalLaxFriedrichs::operator() (lsLocalLaxFriedrichs.hpp:65-241)
-template <int D>
-LSG_HD inline RateOut schemeLLF(const BandView &b, const int32_t c[3], double phi0, int order, const Vel &vel,
+template <int D, class V>
+LSG_HD inline RateOut schemeLLF(const V &b, const int32_t c[3], double phi0, int order, const Vel &vel,
                                 double alphaFactor, double *alphaAcc) {
   double gradPos[D], gradNeg[D];
   double grad = 0., dissipation = 0.;
@@ -1629,7 +1629,7 @@ LSG_HD inline RateOut schemeLLF(const BandView &b, const int32_t c[3], double ph
     LSG_UNROLL
     for (int g = 0; g < G; ++g) llfBoxLocs<D>(b, c, q0 + g, lin, off, l + g * NL);
     double bv[G * NL];
-    b.values<G * NL>(l, bv);
+    b.template values<G * NL>(l, bv);
     LSG_UNROLL
     for (int g = 0; g < G; ++g) {
       const int q = q0 + g;
@@ -1666,7 +1666,7 @@ LSG_HD inline RateOut schemeLLF(const BandView &b, const int32_t c[3], double ph
 // Values of the 3^D box around c, boundary mapped per coordinate of the
 // offset from the centre: box[(ox + 1) + 3 (oy + 1) + 9 (oz + 1)].  All
 // lookups are issued together.
-template <int D> LSG_HD inline void gatherBox(const BandView &b, const int32_t c[3], double *box) {
+template <int D, class V> LSG_HD inline void gatherBox(const V &b, const int32_t c[3], double *box) {
   constexpr int NB = (D == 3) ? 27 : 9;
   BandView::Loc l[NB];
   int64_t off[3][3];
@@ -1685,7 +1685,7 @@ template <int D> LSG_HD inline void gatherBox(const BandView &b, const int32_t c
       l[q] = b.locate(p[0], p[1], p[2]);
     }
   }
-  b.values<NB>(l, box);
+  b.template values<NB>(l, box);
 }
 
 // StencilLocalLaxFriedrichsScalar<T,D,1>::operator()
@@ -1733,8 +1733,8 @@ LSG_HD inline double sllfEpsilon(double baseEps, double lsv) {
   return DN;
 }
 
-template <int D>
-LSG_HD inline RateOut schemeSLLF(const BandView &b, const int32_t c[3], const Vel &vel, double baseNormalEps,
+template <int D, class V>
+LSG_HD inline RateOut schemeSLLF(const V &b, const int32_t c[3], const Vel &vel, double baseNormalEps,
                                  double *finalAlphas, bool &used) {
   constexpr int NB = (D == 3) ? 27 : 9;
   double box[NB];
@@ -1906,8 +1906,8 @@ LSG_HD inline int schemeIdOf(int spatial) {
 // velocity after updateLevelSet's checkDissipation rule (lsAdvect.hpp:738-744,
 // precedence kept) and the raw H - D through `velocity`.  SLLF writes the
 // point's finalAlphas to alphaAcc and sets *sllfUsed when it set them.
-template <int D, int SCHEME>
-LSG_HD inline double ratePoint(const BandView &b, const int32_t c[3], double phi0, const RateParams &rp, const Vel &vel,
+template <int D, int SCHEME, class V>
+LSG_HD inline double ratePoint(const V &b, const int32_t c[3], double phi0, const RateParams &rp, const Vel &vel,
                                const double *globalAlphas, double *alphaAcc, double &velocity,
                                const float *mlp = nullptr, float *io = nullptr, bool *sllfUsed = nullptr,
                                double *dnOut = nullptr, int learnedPhase = 0, const double *stc = nullptr,
@@ -1935,7 +1935,7 @@ LSG_HD inline double ratePoint(const BandView &b, const int32_t c[3], double phi
 
 // Normal of Advect::findGlobalAlphas (lsAdvect.hpp:150-162): phiPos -
 // phiNeg per direction, normalised.
-template <int D> LSG_HD inline void globalAlphaNormal(const BandView &b, const int32_t c[3], double normal[3]) {
+template <int D, class V> LSG_HD inline void globalAlphaNormal(const V &b, const int32_t c[3], double normal[3]) {
   normal[0] = normal[1] = normal[2] = 0.;
   double nm = 0.;
   double st[D][3];
@@ -1950,7 +1950,7 @@ template <int D> LSG_HD inline void globalAlphaNormal(const BandView &b, const i
   for (int k = 0; k < D; ++k) normal[k] *= nm;
 }
 // Per-point alphas of Advect::findGlobalAlphas (lsAdvect.hpp:150-178).
-template <int D> LSG_HD inline void globalAlphaPoint(const BandView &b, const int32_t c[3], const Vel &vel, double *la) {
+template <int D, class V> LSG_HD inline void globalAlphaPoint(const V &b, const int32_t c[3], const Vel &vel, double *la) {
   double normal[3];
   globalAlphaNormal<D>(b, c, normal);
   const double sv = vel.scalar(normal);

@@ -1,0 +1,980 @@
+// Kernels on word bands (lsg_words.hpp), written for CDNA4 (gfx950, wave64).
+//
+// One launch per band operation.  A workgroup takes strips of 16 words dealt
+// round robin over the grid, so that a slab of words with work (a flat part
+// of a surface fills whole layers of the frame) spreads over the chip.
+// First every thread looks at one word: the words with points to evaluate
+// go on a list in LDS, the others are written at once.  Then every wave takes
+// words from the list, lane = point: the y and z neighbours of the 64 points
+// are the same lanes of other words (coalesced value loads at wave-uniform
+// offsets, no per-point decode or rank), the x neighbours are the lanes
+// beside, and the result's bitmaps are wave ballots.  No operation waits on
+// a scan, so nothing else has to be launched for it.
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cstdint>
+
+#include "lsg_block.hpp"
+#include "lsg_words_launch.hpp"
+
+namespace lsg {
+
+static constexpr uint32_t STRIP = 16;
+
+__device__ inline uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ inline uint64_t uni(uint64_t v) { return (uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32); }
+
+// Workgroups of the word kernels: up to 16 strips (256 words, one per
+// thread) each, fewer while that gives 4 workgroups per CU.
+static uint32_t wordGrid(uint32_t nw) {
+  const uint32_t strips = (nw + STRIP - 1) / STRIP;
+  const uint32_t per = std::max(1u, std::min((uint32_t)TPB / STRIP, strips / 1024u));
+  return (strips + per - 1) / per;
+}
+
+// XCD-contiguous index of worker block b of n.
+__device__ inline uint32_t xcdOrder(uint32_t b, uint32_t n) {
+  const uint32_t xcd = b % NUM_XCD, k = b / NUM_XCD;
+  const uint32_t per = n / NUM_XCD, rem = n % NUM_XCD;
+  return xcd * per + (xcd < rem ? xcd : rem) + k;
+}
+
+// The words of a workgroup in rounds of 16 strips (one word per thread);
+// thread-level `first(w, push)` decides whether word w goes on the list with
+// its 64-bit mask, wave-level `each(w, mask)` runs for every listed word.
+template <class First, class Each>
+__device__ __attribute__((always_inline)) inline void forWords(uint32_t nw, uint32_t b, uint32_t nb, First first,
+                                                               Each each) {
+  __shared__ uint32_t listW[TPB];
+  __shared__ uint64_t listM[TPB];
+  __shared__ uint32_t count;
+  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t strips = (nw + STRIP - 1) / STRIP;
+  for (uint32_t j0 = 0; j0 * nb + b < strips; j0 += TPB / STRIP) {
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    const uint32_t strip = (j0 + threadIdx.x / STRIP) * nb + b;
+    const uint32_t w = strip * STRIP + threadIdx.x % STRIP;
+    uint64_t mask = 0;
+    if (strip < strips && w < nw) mask = first(w);
+    const uint64_t has = (uint64_t)__ballot(mask != 0);
+    if (has) {
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(&count, (uint32_t)__builtin_popcountll(has));
+      at = uni(at);
+      if (mask) {
+        const uint32_t i = at + (uint32_t)__builtin_popcountll(has & ((1ull << lane) - 1ull));
+        listW[i] = w;
+        listM[i] = mask;
+      }
+    }
+    __syncthreads();
+    const uint32_t n = count;
+    for (uint32_t i = wid; i < n; i += TPB / 64) each(uni(listW[i]), uni(listM[i]));
+    __syncthreads();
+  }
+}
+
+__global__ void kWordPages(double *pages) {
+  pages[threadIdx.x] = threadIdx.x < 64 ? POS : NEG;
+}
+void launchWordPages(hipStream_t s, double *pages) { kWordPages<<<1, 64 * WORD_PAGES, 0, s>>>(pages); }
+
+// Slot at a byte offset from the first page.
+__device__ inline double slotAt(const double *val, uint32_t off) {
+  return *(const double *)((const char *)(val - 64 * WORD_PAGES) + off);
+}
+__device__ inline void setSlot(double *val, uint32_t off, double v) {
+  *(double *)((char *)(val - 64 * WORD_PAGES) + off) = v;
+}
+// Offset of the slots of word w (bits b): its page if it is uniform.
+__device__ inline uint32_t slotsOf(const WordBits &b, uint64_t valid, uint32_t w) {
+  return uniformWord(b, valid) ? (b.neg ? PAGE_NEG : PAGE_POS) : wordOffset(w);
+}
+__device__ inline uint64_t validOf(const Frame &f, uint32_t w) {
+  return wordValid(f, (int)(w - f.divW.div(w) * (uint32_t)f.wpr));
+}
+__device__ inline double pointOf(const WordBits &q, const double *val, uint32_t w, int bit) {
+  return ((q.def >> bit) & 1ull) ? val[(w << 6) | (uint32_t)bit] : (((q.neg >> bit) & 1ull) ? NEG : POS);
+}
+__device__ inline bool undefinedValue(double v) { return fabs(v) == POS; }
+// Bits and slots of a word from its points' values (one per lane); past the
+// row's end v is POS.
+__device__ inline void putWord(WordBits *wb, double *val, uint32_t w, uint32_t lane, double v) {
+  WordBits r;
+  r.def = (uint64_t)__ballot(!undefinedValue(v));
+  r.neg = (uint64_t)__ballot(v < 0);
+  if (lane == 0) wb[w] = r;
+  val[(w << 6) | lane] = v;
+}
+__device__ inline void putPoint(WordBits *wb, double *val, uint32_t w, double v) {  // the grid-minimum entry
+  wb[w] = WordBits{undefinedValue(v) ? 0ull : 1ull, v < 0 ? 1ull : 0ull};
+  val[w << 6] = v;
+}
+
+__device__ inline void resetStep(WordStep *st, const double *maxDt) {
+  for (int i = threadIdx.x; i < STEP_STAGES * STEP_SLOTS; i += TPB) {
+    (&st->active[0][0])[i] = 0ull;
+    (&st->maxAbs[0][0])[i] = 0ull;
+  }
+  for (int i = threadIdx.x; i < STEP_STAGES * 3 * STEP_SLOTS; i += TPB) (&st->alpha[0][0][0])[i] = 0ull;
+  if (threadIdx.x < STEP_STAGES) st->sllfKey[threadIdx.x] = 0ull;
+  if (threadIdx.x == 0) {
+    st->reframe = 0;
+    st->maxTimeStep = *maxDt;
+  }
+}
+__global__ __launch_bounds__(256) void kWordBegin(WordStep *st, const double *maxDt) { resetStep(st, maxDt); }
+void launchWordBegin(hipStream_t s, WordStep *st, const double *maxDt) { kWordBegin<<<1, TPB, 0, s>>>(st, maxDt); }
+
+// Maximum of a stage's slots (bit patterns of non-negative doubles order
+// like the values), in every lane.
+__device__ inline double slotMax(const unsigned long long *slots) {
+  unsigned long long v = slots[threadIdx.x & 63];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const unsigned long long y = __shfl_xor(v, o, 64);
+    v = (y > v) ? y : v;
+  }
+  return __longlong_as_double((long long)v);
+}
+
+// Whether a word's defined points come close to an open frame edge.
+__device__ inline bool nearEdge(const Frame &f, const GridInfo &g, int D, uint64_t def, int kw, int yr, int zr,
+                                int slack) {
+  bool near = false;
+  if (!g.bounded(0)) {
+    const int lo = kw * 64 + __builtin_ctzll(def), hi = kw * 64 + 63 - __builtin_clzll(def);
+    near = lo < slack || f.ext[0] - 1 - hi < slack;
+  }
+  if (!g.bounded(1)) near = near || yr < slack || f.ext[1] - 1 - yr < slack;
+  if (D > 2 && !g.bounded(2)) near = near || zr < slack || f.ext[2] - 1 - zr < slack;
+  return near;
+}
+
+// The lane beside (DPP wavefront shifts: lane i takes lane i - 1 / i + 1; the
+// end lanes keep their own value).
+__device__ inline double laneBelow(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x138, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, 0x138, 0xf, 0xf, false));
+}
+__device__ inline double laneAbove(double v) {
+  const int lo = __double2loint(v), hi = __double2hiint(v);
+  return __hiloint2double(__builtin_amdgcn_update_dpp(hi, hi, 0x130, 0xf, 0xf, false),
+                          __builtin_amdgcn_update_dpp(lo, lo, 0x130, 0xf, 0xf, false));
+}
+__device__ inline double laneOf(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l), __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+
+// Records of the words a workgroup evaluates: where the slots of the word and
+// of its neighbours are, so that the second phase only loads values.  The
+// words of a round are dealt to the waves (record i to wave i % 4); a wave
+// keeps its records in registers, one per lane, and reads them lane by lane.
+template <int D> struct WordRecords {
+  uint32_t word[TPB];            // last valid bit | ONE_POINT
+  uint32_t self[TPB];            // byte offset of the word's slots
+  uint32_t ref[2 * D - 2][TPB];  // of the neighbour words' slots (ONE_POINT words: | 1 where one point is meant)
+  uint32_t end[2][TPB];          // of the slots below the first and above the last point
+  uint32_t in[TPB];              // of the input word's slots (a page where it is uniform)
+  uint64_t cand[TPB];
+  uint32_t count;
+};
+static constexpr uint32_t ONE_POINT = 256u;
+
+// One band operation.  Workgroup 0 evaluates the grid-minimum entry and, in
+// a step's first operation, resets the step's scalars; the others take the
+// words.
+//
+// The cost of a word is its instructions (about 100, a quarter of them the
+// rule) and one round of 2 D loads; two words are in flight per wave.  A word
+// without points to evaluate costs its share of the first phase only.
+template <int D, int OP>
+__global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb, const double *__restrict__ val,
+                                                 const double *__restrict__ rates, WordBits *__restrict__ owb,
+                                                 double *__restrict__ oval, uint64_t *__restrict__ oact, WordFrame F,
+                                                 GridInfo g, uint32_t nw, WordOpArgs a, WordStep *st) {
+  constexpr bool STAR = OP == W_EXPAND || OP == W_REBUILD || OP == W_UPD_REBUILD;
+  constexpr bool UPD = OP == W_UPD_REBUILD;
+  constexpr bool NEIGHBOURS = OP != W_REDUCE;
+  constexpr int NR = 2 * D - 2;
+  const Frame &f = F.f;
+  double dt = 0.;
+  if (UPD) {
+    double al[3] = {0., 0., 0.};
+    const double m = slotMax(st->maxAbs[a.stage]);
+    if (a.useAlphas)
+      for (int d = 0; d < D; ++d) al[d] = slotMax(st->alpha[a.stage][d]);
+    dt = stageTimeStep(*a.maxDt, a.cfl, m, D, al, a.useAlphas != 0, g.dx);
+  }
+  if (blockIdx.x == 0) {
+    if (UPD && threadIdx.x == 0) st->dt[a.stage] = dt;
+    if (a.begin) resetStep(st, a.begin);
+    if (threadIdx.x == 64) {
+      double r = POS;
+      if (f.base) {
+        double c;
+        r = wordRuleMin<D, OP>(F, wb, val, rates, dt, a.a, a.b, c);
+        if (OP == W_EXPAND && isUndef(c) && r != c) st->conflict = 1;
+      }
+      putPoint(owb, oval, nw, r);
+    }
+    return;
+  }
+  __shared__ WordRecords<D> R;
+  const uint32_t nb = gridDim.x - 1, b = xcdOrder(blockIdx.x - 1, nb);
+  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t lane8 = lane * 8u;
+  const uint32_t strips = (nw + STRIP - 1) / STRIP;
+  uint32_t touched = 0;
+  for (uint32_t j0 = 0; j0 * nb + b < strips; j0 += TPB / STRIP) {
+    if (threadIdx.x == 0) R.count = 0;
+    __syncthreads();
+    const uint32_t strip = (j0 + threadIdx.x / STRIP) * nb + b;
+    const uint32_t w = strip * STRIP + threadIdx.x % STRIP;
+    uint64_t cand = 0;
+    bool listed = false;
+    WordSite<D> s;
+    uint64_t valid = ~0ull;
+    if (strip < strips && w < nw) {
+      if (STAR) {
+        wordSite<D>(wb, F, w, s);
+        bool conflict = false;
+        if (!quietSite<D>(F, s)) cand = starPoints<D, OP == W_EXPAND>(wb, F, w, s, conflict);
+        if (OP == W_EXPAND && conflict) st->conflict = 1;
+        listed = cand != 0;
+        if (UPD && listed) {  // without an active point in its stars the word ends undefined
+          uint64_t act = a.inAct[w];
+          LSG_UNROLL
+          for (int k = 0; k < NR; ++k) act |= s.ref[k].w < nw ? a.inAct[s.ref[k].w] : 1ull;
+          act |= s.below.w < nw ? a.inAct[s.below.w] : 1ull;
+          act |= s.above.w < nw ? a.inAct[s.above.w] : 1ull;
+          if (!act) {
+            const uint64_t neg = s.self.neg;
+            s.self = WordBits{0, neg};
+            valid = wordValid(f, s.kw);
+            // a word of both signs keeps its slots
+            listed = !uniformWord(s.self, valid);
+          }
+        }
+      } else {
+        s.self = wb[w];
+        cand = s.self.def;
+        f.wordRow(w, s.kw, s.yr, s.zr);
+        listed = !uniformWord(s.self, wordValid(f, s.kw));
+        if (listed) wordSite<D>(wb, F, w, s);
+      }
+      if (!listed) {
+        owb[w] = s.self;
+        if (oact) oact[w] = 0ull;
+      } else if (a.count) {
+        touched += (uint32_t)(__builtin_popcountll(cand) + __builtin_popcountll(s.self.def));
+      }
+    }
+    const uint64_t has = (uint64_t)__ballot(listed);
+    if (has) {
+      uint32_t at = 0;
+      if (lane == 0) at = atomicAdd(&R.count, (uint32_t)__builtin_popcountll(has));
+      at = uni(at);
+      if (listed) {
+        const uint32_t i = at + (uint32_t)__builtin_popcountll(has & ((1ull << lane) - 1ull));
+        valid = wordValid(f, s.kw);
+        uint32_t word = s.kw == wordLast(f) ? (uint32_t)rowLastBit(f) : 63u;
+        R.self[i] = wordOffset(w);
+        R.cand[i] = cand;
+        // the input's slots: of the word itself they are the operation's
+        // target too, so a uniform input word is marked by its page here
+        R.in[i] = slotsOf(wb[w], valid, w);
+        if (NEIGHBOURS) {
+          LSG_UNROLL
+          for (int k = 0; k < NR; ++k) {
+            const WordRef r = s.ref[k];
+            uint32_t off = slotsOf(s.bits[k], valid, r.w);
+            if (r.bit >= 0) {  // one point outside the frame's rows
+              const bool neg = (s.bits[k].neg >> r.bit) & 1ull;
+              off = neg ? PAGE_NEG : PAGE_POS;
+              if ((s.bits[k].def >> r.bit) & 1ull) {
+                off = (wordOffset(r.w) + (uint32_t)r.bit * 8u) | 1u;
+                word |= ONE_POINT;
+              }
+            }
+            R.ref[k][i] = off;
+          }
+          R.end[0][i] = s.belowDef ? wordOffset(s.below.w) + (uint32_t)s.below.bit * 8u : (s.belowNeg ? PAGE_NEG : PAGE_POS);
+          R.end[1][i] = s.aboveDef ? wordOffset(s.above.w) + (uint32_t)s.above.bit * 8u : (s.aboveNeg ? PAGE_NEG : PAGE_POS);
+        }
+        R.word[i] = word;
+      }
+    }
+    __syncthreads();
+    const uint32_t n = R.count;
+    const uint32_t mine = n > wid ? (n - wid + TPB / 64 - 1) / (TPB / 64) : 0u;
+    if (mine) {
+      // this wave's records, one per lane
+      const uint32_t ri = lane < mine ? lane * (TPB / 64) + wid : wid;
+      const uint32_t rWord = R.word[ri], rSelf = R.self[ri], rIn = R.in[ri];
+      const uint64_t rCand = R.cand[ri];
+      uint32_t rRef[NR], rEnd[2];
+      if (NEIGHBOURS) {
+        LSG_UNROLL
+        for (int k = 0; k < NR; ++k) rRef[k] = R.ref[k][ri];
+        rEnd[0] = R.end[0][ri];
+        rEnd[1] = R.end[1][ri];
+      }
+      uint32_t dLo = 0, dHi = 0, nLo = 0, nHi = 0, aLo = 0, aHi = 0;  // results, record j in lane j
+      struct Star {
+        double v[2 * D];
+      };
+      auto at = [&](uint32_t x, uint32_t j) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)j); };
+      auto put = [&](uint32_t j, double o) {
+        setSlot(oval, at(rSelf, j) + lane8, o);
+        const uint64_t def = (uint64_t)__ballot(!undefinedValue(o));
+        const uint64_t neg = (uint64_t)__ballot(o < 0) & (~0ull >> (63u - (at(rWord, j) & 63u)));
+        dLo = lane == j ? (uint32_t)def : dLo;
+        dHi = lane == j ? (uint32_t)(def >> 32) : dHi;
+        nLo = lane == j ? (uint32_t)neg : nLo;
+        nHi = lane == j ? (uint32_t)(neg >> 32) : nHi;
+        if (oact) {
+          const uint64_t act = (uint64_t)__ballot(fabs(o) <= 0.5);
+          aLo = lane == j ? (uint32_t)act : aLo;
+          aHi = lane == j ? (uint32_t)(act >> 32) : aHi;
+        }
+      };
+      auto load = [&](uint32_t j, Star &z) {
+        z.v[0] = slotAt(val, at(rIn, j) + lane8);
+        if (NEIGHBOURS) {
+          if (at(rWord, j) & ONE_POINT) {
+            LSG_UNROLL
+            for (int k = 0; k < NR; ++k) {
+              const uint32_t o = at(rRef[k], j);
+              z.v[1 + k] = slotAt(val, (o & ~7u) + ((o & 1u) ? 0u : lane8));
+            }
+          } else {
+            LSG_UNROLL
+            for (int k = 0; k < NR; ++k) z.v[1 + k] = slotAt(val, at(rRef[k], j) + lane8);
+          }
+          const uint32_t e0 = at(rEnd[0], j), e1 = at(rEnd[1], j);
+          z.v[2 * D - 1] = slotAt(val, lane < 32u ? e0 : e1);
+        }
+      };
+      auto update = [&](uint32_t j, Star &z) {  // updateLevelSet's rule on the star
+        auto one = [&](double v, uint32_t off) {
+          const bool act = fabs(v) <= 0.5;
+          double r = 0.;
+          if (__any(act)) r = slotAt(rates, off);
+          return ruleUpdate(v, dt, r);
+        };
+        z.v[0] = one(z.v[0], at(rIn, j) + lane8);
+        const bool single = at(rWord, j) & ONE_POINT;
+        LSG_UNROLL
+        for (int k = 0; k < NR; ++k) {
+          const uint32_t o = at(rRef[k], j);
+          z.v[1 + k] = one(z.v[1 + k], (single && (o & 1u)) ? (o & ~7u) : (o & ~7u) + lane8);
+        }
+        const uint32_t e0 = at(rEnd[0], j), e1 = at(rEnd[1], j);
+        z.v[2 * D - 1] = one(z.v[2 * D - 1], lane < 32u ? e0 : e1);
+      };
+      auto finish = [&](uint32_t j, Star &z) {
+        if (UPD) update(j, z);
+        const double c = z.v[0];
+        const uint64_t c64 = (uint64_t)at((uint32_t)rCand, j) | ((uint64_t)at((uint32_t)(rCand >> 32), j) << 32);
+        double nbv[2 * D];
+        if (NEIGHBOURS) {
+          LSG_UNROLL
+          for (int d = 1; d < D; ++d) {
+            nbv[d] = z.v[2 * d - 1];
+            nbv[D + d] = z.v[2 * d];
+          }
+          const double vm = laneOf(z.v[2 * D - 1], 0), vp = laneOf(z.v[2 * D - 1], 63);
+          const double above = laneAbove(c), below = laneBelow(c);
+          nbv[0] = lane == (at(rWord, j) & 63u) ? vp : above;
+          nbv[D] = lane == 0 ? vm : below;
+        }
+        const double r = wordRule<D, OP>(c, nbv, a.a, a.b);
+        put(j, __builtin_amdgcn_inverse_ballot_w64(c64) ? r : c);
+      };
+      for (uint32_t j = 0; j < mine; j += 2) {
+        const uint32_t k = j + 1 < mine ? j + 1 : j;  // the last of an odd number twice, with the same result
+        Star x, y;
+        load(j, x);
+        load(k, y);
+        finish(j, x);
+        finish(k, y);
+      }
+      if (lane < mine) {
+        const uint32_t u = (rSelf >> 9) - WORD_PAGES;
+        const WordBits o{(uint64_t)dLo | ((uint64_t)dHi << 32), (uint64_t)nLo | ((uint64_t)nHi << 32)};
+        owb[u] = o;
+        if (oact) oact[u] = (uint64_t)aLo | ((uint64_t)aHi << 32);
+        if (a.slack > 0 && o.def) {
+          int32_t kw, yr, zr;
+          f.wordRow(u, kw, yr, zr);
+          if (nearEdge(f, g, D, o.def, kw, yr, zr, a.slack)) st->reframe = 1;
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (a.count && touched) atomicAdd(&st->starBytes[b % STEP_SLOTS], 8.0 * (double)touched);
+}
+
+template <int D>
+static void wordStar(hipStream_t s, int op, const WordBufs &in, const WordBufs &out, const Frame &f, const GridInfo &g,
+                     const WordOpArgs &a, WordStep *st) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  const uint32_t grid = wordGrid(nw) + 1;
+  WordFrame F;
+  F.init(f, g);
+#define LSG_WORD(OP) \
+  kWordStar<D, OP><<<grid, TPB, 0, s>>>(in.wb, in.val, a.rates, out.wb, out.val, a.act, F, g, nw, a, st)
+  switch (op) {
+  case W_EXPAND: LSG_WORD(W_EXPAND); break;
+  case W_REBUILD: LSG_WORD(W_REBUILD); break;
+  case W_UPD_REBUILD: LSG_WORD(W_UPD_REBUILD); break;
+  case W_REDUCE: LSG_WORD(W_REDUCE); break;
+  case W_PRUNE: LSG_WORD(W_PRUNE); break;
+  default: LSG_WORD(W_PRUNE_RSZ); break;
+  }
+#undef LSG_WORD
+}
+void launchWordStar(hipStream_t s, int D, int op, const WordBufs &in, const WordBufs &out, const Frame &f,
+                    const GridInfo &g, const WordOpArgs &a, WordStep *st) {
+  if (D == 2) wordStar<2>(s, op, in, out, f, g, a, st);
+  else wordStar<3>(s, op, in, out, f, g, a, st);
+}
+
+// BooleanOperation's comparators (pointwise; the grid-minimum word is one of
+// the words here).
+__global__ __launch_bounds__(256) void kWordBool(const WordBits *__restrict__ awb, const double *__restrict__ aval,
+                                                 const WordBits *__restrict__ bwb, const double *__restrict__ bval,
+                                                 WordBits *__restrict__ owb, double *__restrict__ oval, Frame f,
+                                                 uint32_t nw, int kind, double wT, double wS) {
+  const uint32_t lane = threadIdx.x & 63u;
+  forWords(
+      nw + 1, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        const WordBits x = awb[w], y = bwb[w];
+        const uint64_t valid = w < nw ? validOf(f, w) : 1ull;
+        const bool ux = uniformWord(x, valid), uy = uniformWord(y, valid);
+        if (ux && uy) {
+          owb[w] = WordBits{0, boolNeg(kind, x.neg, y.neg)};
+          return 0ull;
+        }
+        // the slots of both words
+        return ((uint64_t)slotsOf(y, valid, w) << 32) | (uint64_t)slotsOf(x, valid, w) | 1ull;
+      },
+      [&](uint32_t w, uint64_t slots) {
+        const double p = slotAt(aval, ((uint32_t)slots & ~7u) + lane * 8u);
+        const double q = slotAt(bval, (uint32_t)(slots >> 32) + lane * 8u);
+        double o = ruleBoolean(kind, p, q, wT, wS);
+        const uint64_t valid = w < nw ? validOf(f, w) : 1ull;
+        o = __builtin_amdgcn_inverse_ballot_w64(valid) ? o : POS;
+        putWord(owb, oval, w, lane, o);
+      });
+}
+void launchWordBoolean(hipStream_t s, const WordBufs &A, const WordBufs &B, const WordBufs &out, const Frame &f,
+                       int kind, double wTarget, double wSource) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordBool<<<wordGrid(nw + 1), TPB, 0, s>>>(A.wb, A.val, B.wb, B.val, out.wb, out.val, f, nw, kind, wTarget, wSource);
+}
+
+// ------------------------------------------------------------- rates ----
+
+// Active points (|phi| <= 1/2) of a band, one bit per point: written by the
+// operation that made the band (WordOpArgs::act), or here.
+__global__ __launch_bounds__(256) void kWordActive(const WordBits *__restrict__ wb, const double *__restrict__ val,
+                                                   uint64_t *__restrict__ act, uint32_t nw) {
+  const uint32_t lane = threadIdx.x & 63u;
+  forWords(
+      nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        const uint64_t d = wb[w].def;
+        if (!d) act[w] = 0ull;
+        return d;
+      },
+      [&](uint32_t w, uint64_t) {
+        const uint64_t m = (uint64_t)__ballot(fabs(val[(w << 6) | lane]) <= 0.5);
+        if (lane == 0) act[w] = m;
+      });
+}
+void launchWordActive(hipStream_t s, const WordBufs &b, const Frame &f, uint64_t *act) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordActive<<<wordGrid(nw), TPB, 0, s>>>(b.wb, b.val, act, nw);
+}
+
+// The active points of the workgroup's words, 256 words at a time, handed to
+// `fn` one per lane in full waves (the rest below a wave waits for the next
+// words), so that the scheme runs with idle lanes only once.  fn(p) gets the
+// frame position.  The list holds 64 words' worth of points; fuller rounds
+// run in parts.
+static constexpr uint32_t ACTIVE_LIST = 4096;
+// words dealt to the workgroups in pairs: the words of a flat part of the
+// surface are full and lie side by side, and a strip of 16 of them would be
+// 16 waves of work for one workgroup beside workgroups with one
+static constexpr uint32_t PAIR = 2;
+template <class Fn>
+__device__ __attribute__((always_inline)) inline void forActivePoints(const uint64_t *__restrict__ act, uint32_t nw,
+                                                                      uint32_t b, uint32_t nb, Fn fn) {
+  __shared__ uint32_t list[ACTIVE_LIST + 64];
+  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t pairs = (nw + PAIR - 1) / PAIR;
+  uint32_t held = 0;  // points left from the round before, at the list's start
+  for (uint32_t j0 = 0; j0 * nb + b < pairs; j0 += TPB / PAIR) {
+    const uint32_t pair = (j0 + threadIdx.x / PAIR) * nb + b;
+    const uint32_t w = pair * PAIR + threadIdx.x % PAIR;
+    const uint64_t m = (pair < pairs && w < nw) ? act[w] : 0ull;
+    uint32_t total;
+    const uint32_t first = blockExclusiveScan((uint32_t)__builtin_popcountll(m), total);
+    const bool lastWords = (j0 + TPB / PAIR) * nb + b >= pairs;
+    for (uint32_t done = 0;;) {  // the points [done, done + room) of this round's
+      const uint32_t room = ACTIVE_LIST;
+      const uint32_t part = total - done < room ? total - done : room;
+      const bool last = lastWords && done + part == total;
+      uint64_t has = (uint64_t)__ballot(m != 0ull && first + 64u > done && first < done + part);
+      while (has) {  // lane = point of the word owned by lane j
+        const int j = __builtin_ctzll(has);
+        has &= has - 1ull;
+        const uint64_t mj = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)m, j) |
+                            ((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(m >> 32), j) << 32);
+        const uint32_t fj = (uint32_t)__builtin_amdgcn_readlane((int)first, j);
+        const uint32_t wj = (uint32_t)__builtin_amdgcn_readlane((int)w, j);
+        const uint32_t at = fj + (uint32_t)__builtin_popcountll(mj & ((1ull << lane) - 1ull)) - done;  // wraps below
+        if (((mj >> lane) & 1ull) && at < part) list[held + at] = (wj << 6) | lane;
+      }
+      __syncthreads();
+      const uint32_t n = held + part;
+      const uint32_t take = last ? n : n / 64u * 64u;
+      for (uint32_t i = wid * 64u + lane; i < take; i += TPB) fn(list[i]);
+      __syncthreads();
+      held = n - take;
+      uint32_t p = 0;
+      if (threadIdx.x < held) p = list[take + threadIdx.x];
+      __syncthreads();
+      if (threadIdx.x < held) list[threadIdx.x] = p;
+      __syncthreads();
+      done += part;
+      if (done >= total) break;
+    }
+  }
+}
+
+__device__ inline void blockMaxSlot(double v, unsigned long long *slots) {
+  blockMaxAtomic((unsigned long long)__double_as_longlong(v), &slots[blockIdx.x % STEP_SLOTS]);
+}
+
+template <int D>
+__global__ __launch_bounds__(256) void kWordAlphas(WordView v, const uint64_t *__restrict__ act, uint32_t nw,
+                                                   RateParams rp, int stage, WordStep *st) {
+  const Vel vel = velOf(rp);
+  double la[3] = {0., 0., 0.};
+  forActivePoints(act, nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](uint32_t p) {
+    int32_t c[3];
+    v.coords(p, c);
+    globalAlphaPoint<D>(v, c, vel, la);
+  });
+  for (int d = 0; d < D; ++d) blockMaxSlot(la[d], st->alpha[stage][d]);
+}
+
+// Advect::integrateTime for one level set (lsAdvect.hpp:495-593): the stage
+// velocity of every active point at its slot of `rates`, the maxima in the
+// step's slots.
+template <int D, int SCHEME>
+__global__ __launch_bounds__(256) void kWordRates(WordView v, const uint64_t *__restrict__ act, uint32_t nw,
+                                                  RateParams rp, double *__restrict__ rates,
+                                                  const double *__restrict__ box, int stage, int count, WordStep *st) {
+  const Vel vel = velOf(rp);
+  double ga[3] = {0., 0., 0.}, la[3] = {0., 0., 0.};
+  if (SCHEME == S_LF)
+    for (int d = 0; d < D; ++d) ga[d] = slotMax(st->alpha[stage][d]);
+  double lmax = 0.;
+  unsigned long long points = 0, key = 0;
+  forActivePoints(act, nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](uint32_t p) {
+    ++points;
+    double velocity;
+    bool used = false, outside = false;
+    rates[p] = wordRatePoint<D, SCHEME>(v, p, rp, vel, ga, la, velocity, used, box, &outside);
+    if (SCHEME == S_LLF_BOX && outside) st->conflict = 1;
+    if (SCHEME == S_SLLF && used && (unsigned long long)p + 1ull > key) key = (unsigned long long)p + 1ull;
+    const double m = fabs(velocity);
+    if (lmax < m) lmax = m;
+  });
+  blockMaxSlot(lmax, st->maxAbs[stage]);
+  if (SCHEME == S_LLLF || SCHEME == S_LLF || SCHEME == S_LLFA || SCHEME == S_LLF_BOX)
+    for (int d = 0; d < D; ++d) blockMaxSlot(la[d], st->alpha[stage][d]);
+  if (SCHEME == S_SLLF) blockMaxAtomic(key, &st->sllfKey[stage]);
+  const unsigned long long t = blockSumU64(points);
+  if (threadIdx.x == 0 && t) {
+    atomicAdd(&st->active[stage][blockIdx.x % STEP_SLOTS], t);
+    if (count) atomicAdd(&st->rateBytes[blockIdx.x % STEP_SLOTS], 8.0 * (double)t);
+  }
+  if (count) {  // every defined point of the band read once
+    unsigned long long d = 0;
+    for (uint32_t w = blockIdx.x * TPB + threadIdx.x; w < nw; w += gridDim.x * TPB)
+      d += (unsigned long long)__builtin_popcountll(v.wb[w].def);
+    d = blockSumU64(d);
+    if (threadIdx.x == 0 && d) atomicAdd(&st->rateBytes[blockIdx.x % STEP_SLOTS], 8.0 * (double)d);
+  }
+}
+
+// Box alphas (boxAlphas) of every point in the 3^D box of an active point, in
+// words: computed once per point here where the scheme's own loop computes
+// the normal of each of the 3^D box points of every active point.
+template <int D>
+__global__ __launch_bounds__(256) void kWordBoxAlphas(WordView v, const uint64_t *__restrict__ act, WordFrame F,
+                                                      uint32_t nw, RateParams rp, double *__restrict__ box) {
+  const Frame &f = F.f;
+  const uint32_t lane = threadIdx.x & 63u;
+  const Vel vel = velOf(rp);
+  forWords(
+      nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        int32_t kw, yr, zr;
+        f.wordRow(w, kw, yr, zr);
+        const int wl = wordLast(f), lb = rowLastBit(f);
+        // the words beside this one along x whose end points see it
+        uint32_t wm = w, wp = w;
+        int bm = -1, bp = -1;
+        const WordRef m = edgeRef(F, w, kw, zr * f.ext[1] + yr, -1), p = edgeRef(F, w, kw, zr * f.ext[1] + yr, 1);
+        if (m.w < nw && (kw > 0 || F.first[0] >= 0)) wm = m.w, bm = m.bit;
+        if (p.w < nw && (kw < wl || F.last[0] < f.ext[0])) wp = p.w, bp = p.bit;
+        uint64_t any = 0, ends = 0;
+        LSG_UNROLL
+        for (int z = (D == 3 ? -1 : 0); z <= (D == 3 ? 1 : 0); ++z) {
+          const int32_t zz = z == 0 ? zr : F.step(2, zr, z);
+          LSG_UNROLL
+          for (int y = -1; y <= 1; ++y) {
+            const int32_t yy = y == 0 ? yr : F.step(1, yr, y);
+            if (zz < 0 || zz >= f.ext[2] || yy < 0 || yy >= f.ext[1]) continue;
+            const int32_t d = ((zz - zr) * f.ext[1] + (yy - yr)) * f.wpr;
+            any |= act[(uint32_t)((int32_t)w + d)];
+            if (bm >= 0) ends |= act[(uint32_t)((int32_t)wm + d)] >> bm & 1ull;
+            if (bp >= 0) ends |= act[(uint32_t)((int32_t)wp + d)] >> bp & 1ull;
+          }
+        }
+        (void)lb;
+        return any | ends;
+      },
+      [&](uint32_t w, uint64_t) {
+        int32_t kw, yr, zr;
+        f.wordRow(w, kw, yr, zr);
+        const uint64_t valid = wordValid(f, kw);
+        double bv[2 * D + 1];
+        const uint32_t off = slotsOf(v.wb[w], valid, w);
+        const double c = slotAt(v.val, off + lane * 8u);
+        bv[2 * D] = c;
+        LSG_UNROLL
+        for (int d = 1; d < D; ++d)
+          LSG_UNROLL
+          for (int k = 0; k < 2; ++k) {
+            const WordRef r = stepRef(F, w, yr, zr, d, k ? -1 : 1);
+            const WordBits q = v.wb[r.w];
+            bv[d + k * D] = r.bit < 0 ? slotAt(v.val, slotsOf(q, valid, r.w) + lane * 8u) : pointOf(q, v.val, r.w, r.bit);
+          }
+        const int32_t row = zr * f.ext[1] + yr;
+        const WordRef m = edgeRef(F, w, kw, row, -1), p = edgeRef(F, w, kw, row, 1);
+        const double vm = pointOf(v.wb[m.w], v.val, m.w, m.bit), vp = pointOf(v.wb[p.w], v.val, p.w, p.bit);
+        const double above = laneAbove(c), below = laneBelow(c);
+        const int top = kw == wordLast(f) ? rowLastBit(f) : 63;
+        bv[0] = (int)lane == top ? vp : above;
+        bv[D] = lane == 0 ? vm : below;
+        double t[D];
+        boxAlphas<D>(bv, v.g.dx, vel, t);
+        LSG_UNROLL
+        for (int k = 0; k < D; ++k) box[boxSlot<D>((w << 6) | lane, k)] = t[k];
+      });
+}
+
+// The alphas of the stencil scheme's last point (HRLE order), evaluated
+// again (kSllfAlphas).
+template <int D> __global__ void kWordSllfAlphas(WordView v, RateParams rp, int stage, WordStep *st) {
+  const unsigned long long key = st->sllfKey[stage];
+  double fa[3] = {0., 0., 0.};
+  if (key) {
+    int32_t c[3];
+    v.coords((uint32_t)(key - 1ull), c);
+    bool used = false;
+    (void)schemeSLLF<D>(v, c, velOf(rp), rp.sllfBaseEps, fa, used);
+  }
+  for (int d = 0; d < 3; ++d) st->alpha[stage][d][0] = (unsigned long long)__double_as_longlong(fa[d]);
+}
+
+// Workgroups of the passes over active points: 256 words each from 4 per CU on.
+static uint32_t activeGrid(uint32_t nw) {
+  return std::min(4096u, std::max(std::min(1024u, (nw + PAIR - 1) / PAIR), (nw + TPB - 1) / TPB));
+}
+
+void launchWordAlphas(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
+                      const uint64_t *act, int stage, WordStep *st) {
+  const WordView v{b.wb, b.val, f, g};
+  const uint32_t nw = (uint32_t)f.nwords;
+  if (D == 2) kWordAlphas<2><<<activeGrid(nw), TPB, 0, s>>>(v, act, nw, rp, stage, st);
+  else kWordAlphas<3><<<activeGrid(nw), TPB, 0, s>>>(v, act, nw, rp, stage, st);
+}
+
+template <int D>
+static void wordRates(hipStream_t s, const WordView &v, const uint64_t *act, uint32_t nw, const RateParams &rp,
+                      double *rates, double *box, int stage, int count, WordStep *st) {
+  const uint32_t grid = activeGrid(nw);
+#define LSG_WR(S) kWordRates<D, S><<<grid, TPB, 0, s>>>(v, act, nw, rp, rates, box, stage, count, st)
+  switch (schemeIdOf(rp.spatial)) {
+  case S_EO: LSG_WR(S_EO); break;
+  case S_WENO5: LSG_WR(S_WENO5); break;
+  case S_LF: LSG_WR(S_LF); break;
+  case S_LLLF: LSG_WR(S_LLLF); break;
+  case S_LLFA: LSG_WR(S_LLFA); break;
+  case S_LLF:
+    if (box) {
+      WordFrame F;
+      F.init(v.f, v.g);
+      kWordBoxAlphas<D><<<wordGrid(nw), TPB, 0, s>>>(v, act, F, nw, rp, box);
+      LSG_WR(S_LLF_BOX);
+    } else {
+      LSG_WR(S_LLF);
+    }
+    break;
+  case S_SLLF: LSG_WR(S_SLLF); break;
+  default: LSG_WR(S_WENO3); break;
+  }
+#undef LSG_WR
+}
+void launchWordRates(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
+                     const uint64_t *act, double *rates, double *box, int stage, int count, WordStep *st,
+                     hipEvent_t e0, hipEvent_t e1, bool externalEvents) {
+  const WordView v{b.wb, b.val, f, g};
+  const uint32_t nw = (uint32_t)f.nwords;
+  if (e0) (void)hipEventRecordWithFlags(e0, s, externalEvents ? hipEventRecordExternal : hipEventRecordDefault);
+  if (D == 2) wordRates<2>(s, v, act, nw, rp, rates, box, stage, count, st);
+  else wordRates<3>(s, v, act, nw, rp, rates, box, stage, count, st);
+  if (e1) (void)hipEventRecordWithFlags(e1, s, externalEvents ? hipEventRecordExternal : hipEventRecordDefault);
+  if (schemeIdOf(rp.spatial) == S_SLLF) {
+    if (D == 2) kWordSllfAlphas<2><<<1, 1, 0, s>>>(v, rp, stage, st);
+    else kWordSllfAlphas<3><<<1, 1, 0, s>>>(v, rp, stage, st);
+  }
+}
+
+// ------------------------------------------------------- conversions ----
+
+__global__ __launch_bounds__(256) void kWordImport(const uint64_t *__restrict__ bits, const uint32_t *__restrict__ pre,
+                                                   const double *__restrict__ val, WordBits *__restrict__ owb,
+                                                   double *__restrict__ oval, Frame f, uint32_t nw) {
+  const uint32_t lane = threadIdx.x & 63u;
+  const uint32_t base = (uint32_t)f.base;
+  if (blockIdx.x == 0 && threadIdx.x == 0) putPoint(owb, oval, nw, base ? val[0] : POS);
+  forWords(
+      nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        const uint64_t S = bits[w];
+        if (!S) owb[w] = WordBits{0, runValueAt(val, 0ull, base + pre[w], 0) < 0 ? validOf(f, w) : 0ull};
+        return S;
+      },
+      [&](uint32_t w, uint64_t S) {
+        double v = runValueAt(val, S, base + pre[w], (int)lane);
+        if (!((S >> lane) & 1ull)) v = v < 0 ? NEG : POS;
+        if (!__builtin_amdgcn_inverse_ballot_w64(validOf(f, w))) v = POS;
+        putWord(owb, oval, w, lane, v);
+      });
+}
+void launchWordImport(hipStream_t s, const BandBufs &in, const WordBufs &out, const Frame &f) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordImport<<<wordGrid(nw), TPB, 0, s>>>(in.bits, in.pre, in.val, out.wb, out.val, f, nw);
+}
+
+// Canonical run list of a word band, in two kernels over contiguous chunks:
+// start bits with their counts, then prefix counts and entries.
+__global__ __launch_bounds__(256) void kWordCount(const WordBits *__restrict__ wb, Frame f, uint32_t nw,
+                                                  uint64_t *__restrict__ bits, uint32_t *__restrict__ partials) {
+  uint32_t lo, hi;
+  blockChunk(nw, lo, hi);
+  uint32_t acc = 0;
+  for (uint32_t w = lo + threadIdx.x; w < hi; w += TPB) {
+    const uint64_t S = startsOfWord(wb, f, w);
+    bits[w] = S;
+    acc += (uint32_t)__builtin_popcountll(S);
+  }
+  const uint32_t t = blockSum(acc);
+  if (threadIdx.x == 0) partials[logicalBlock()] = t;
+}
+__global__ __launch_bounds__(256) void kWordEmit(const WordBits *__restrict__ wb, const double *__restrict__ wval,
+                                                 Frame f, uint32_t nw, const uint32_t *__restrict__ partials,
+                                                 uint64_t *__restrict__ bits, uint32_t *__restrict__ pre,
+                                                 double *__restrict__ val, uint32_t *__restrict__ pos, uint32_t *nOut,
+                                                 uint32_t *total, size_t cap) {
+  __shared__ uint64_t tileS[TPB];
+  __shared__ uint32_t tileP[TPB];
+  uint32_t lo, hi;
+  blockChunk(nw, lo, hi);
+  uint32_t off = blockOffset(partials);
+  const uint32_t base = (uint32_t)f.base;
+  const int lane = (int)(threadIdx.x & 63u);
+  if (base && logicalBlock() == 0 && threadIdx.x == 0) {
+    const WordBits m = wb[nw];
+    val[0] = (m.def & 1ull) ? wval[(size_t)nw << 6] : ((m.neg & 1ull) ? NEG : POS);
+    pos[0] = POS_NONE;
+  }
+  for (uint32_t t = lo; t < hi; t += TPB) {
+    const uint32_t w = t + threadIdx.x;
+    const uint64_t S = w < hi ? bits[w] : 0ull;
+    uint32_t tot;
+    const uint32_t p = off + blockExclusiveScan((uint32_t)__builtin_popcountll(S), tot);
+    if (w < hi) pre[w] = p;
+    tileS[threadIdx.x] = S;
+    tileP[threadIdx.x] = p;
+    __syncthreads();
+    const uint32_t n = hi - t < (uint32_t)TPB ? hi - t : (uint32_t)TPB;
+    for (uint32_t i = threadIdx.x >> 6; i < n; i += TPB / 64) {
+      const uint64_t s = uni(tileS[i]);
+      if (!s) continue;
+      const uint32_t u = t + i;
+      if ((s >> lane) & 1ull) {
+        const size_t q = (size_t)base + tileP[i] + (uint32_t)__builtin_popcountll(s & ((1ull << lane) - 1ull));
+        if (q < cap) {
+          const WordBits b = wb[u];
+          val[q] = pointOf(b, wval, u, lane);
+          pos[q] = (u << 6) | (uint32_t)lane;
+        }
+      }
+    }
+    __syncthreads();
+    off += tot;
+  }
+  if (logicalBlock() == gridDim.x - 1 && threadIdx.x == 0) {
+    bits[nw] = 0;
+    pre[nw] = off;
+    const size_t all = (size_t)base + off;
+    *total = (uint32_t)all;
+    *nOut = (uint32_t)(all < cap ? all : cap);
+  }
+}
+void launchWordExport(hipStream_t s, const WordBufs &in, BandBufs &out, const Frame &f, const GridInfo &,
+                      uint32_t *partials, uint32_t *total) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  // 64-word chunks at least (blockChunk), at most the partials' capacity
+  const uint32_t grid = std::min<uint32_t>(SCAN_BLOCKS_MAX, std::max<uint32_t>(8u, nw / 64));
+  kWordCount<<<grid, TPB, 0, s>>>(in.wb, f, nw, out.bits, partials);
+  kWordEmit<<<grid, TPB, 0, s>>>(in.wb, in.val, f, nw, partials, out.bits, out.pre, out.val, out.pos, out.n, total,
+                                 out.cap);
+}
+
+__global__ __launch_bounds__(256) void kWordCopy(const WordBits *__restrict__ wb, const double *__restrict__ val,
+                                                 WordBits *__restrict__ owb, double *__restrict__ oval, Frame f,
+                                                 uint32_t nw) {
+  const uint32_t lane = threadIdx.x & 63u;
+  forWords(
+      nw + 1, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        const WordBits b = wb[w];
+        owb[w] = b;
+        return uniformWord(b, w < nw ? validOf(f, w) : 0ull) ? 0ull : 1ull;
+      },
+      [&](uint32_t w, uint64_t) { oval[(w << 6) | lane] = val[(w << 6) | lane]; });
+}
+void launchWordCopy(hipStream_t s, const WordBufs &in, const WordBufs &out, const Frame &f) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordCopy<<<wordGrid(nw + 1), TPB, 0, s>>>(in.wb, in.val, out.wb, out.val, f, nw);
+}
+
+__global__ __launch_bounds__(256) void kWordReframe(WordView v, WordBits *__restrict__ owb, double *__restrict__ oval,
+                                                    Frame fo, uint32_t nwo) {
+  const uint32_t lane = threadIdx.x & 63u;
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    putPoint(owb, oval, nwo, fo.base ? v.value(v.g.lo[0], v.g.lo[1], v.g.lo[2]) : POS);
+  forWords(
+      nwo, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](uint32_t) -> uint64_t { return 1ull; },
+      [&](uint32_t w, uint64_t) {
+        int32_t kw, yr, zr;
+        fo.wordRow(w, kw, yr, zr);
+        double r = POS;
+        if ((wordValid(fo, kw) >> lane) & 1ull) r = v.value(kw * 64 + (int)lane + fo.o[0], yr + fo.o[1], zr + fo.o[2]);
+        putWord(owb, oval, w, lane, r);
+      });
+}
+void launchWordReframe(hipStream_t s, const WordBufs &in, const Frame &f, const GridInfo &g, const WordBufs &out,
+                       const Frame &fo) {
+  const uint32_t nwo = (uint32_t)fo.nwords;
+  kWordReframe<<<wordGrid(nwo), TPB, 0, s>>>(WordView{in.wb, in.val, f, g}, out.wb, out.val, fo, nwo);
+}
+
+__global__ void kWordStatsInit(uint32_t *count, int32_t *bbox, const WordStep *st, uint32_t *conflict) {
+  *conflict = st ? st->conflict : 0u;
+  *count = 0;
+  for (int d = 0; d < 3; ++d) {
+    bbox[d] = INT32_MAX;
+    bbox[3 + d] = INT32_MIN;
+  }
+}
+__global__ __launch_bounds__(256) void kWordStats(const WordBits *__restrict__ wb, Frame f, uint32_t nw,
+                                                  uint32_t *count, int32_t *bbox) {
+  __shared__ int32_t smn[3], smx[3];
+  if (threadIdx.x < 3) {
+    smn[threadIdx.x] = INT32_MAX;
+    smx[threadIdx.x] = INT32_MIN;
+  }
+  __syncthreads();
+  uint32_t c = 0;
+  int32_t mn[3] = {INT32_MAX, INT32_MAX, INT32_MAX}, mx[3] = {INT32_MIN, INT32_MIN, INT32_MIN};
+  for (uint32_t w = blockIdx.x * TPB + threadIdx.x; w < nw; w += gridDim.x * TPB) {
+    c += (uint32_t)__builtin_popcountll(wb[w].def);
+    const uint64_t S = startsOfWord(wb, f, w);
+    if (!S) continue;
+    int32_t kw, r[3];
+    f.wordRow(w, kw, r[1], r[2]);
+    const int32_t a = kw * 64 + __builtin_ctzll(S), z = kw * 64 + 63 - __builtin_clzll(S);
+    mn[0] = a < mn[0] ? a : mn[0];
+    mx[0] = z > mx[0] ? z : mx[0];
+    for (int d = 1; d < 3; ++d) {
+      mn[d] = r[d] < mn[d] ? r[d] : mn[d];
+      mx[d] = r[d] > mx[d] ? r[d] : mx[d];
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0 && f.base && (wb[nw].def & 1ull)) ++c;
+  for (int d = 0; d < 3; ++d)
+    if (mn[d] <= mx[d]) {
+      atomicMin(&smn[d], mn[d]);
+      atomicMax(&smx[d], mx[d]);
+    }
+  const uint32_t t = blockSum(c);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (t) atomicAdd(count, t);
+    for (int d = 0; d < 3; ++d)
+      if (smn[d] <= smx[d]) {
+        atomicMin(&bbox[d], smn[d]);
+        atomicMax(&bbox[3 + d], smx[d]);
+      }
+  }
+}
+void launchWordStats(hipStream_t s, const WordBufs &b, const Frame &f, uint32_t *outCount, int32_t *bbox,
+                     const WordStep *st, uint32_t *conflict) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordStatsInit<<<1, 1, 0, s>>>(outCount, bbox, st, conflict);
+  kWordStats<<<std::min(512u, std::max(1u, nw / TPB)), TPB, 0, s>>>(b.wb, f, nw, outCount, bbox);
+}
+
+// BooleanOperation INVERT: values negated, signs swapped.
+__global__ __launch_bounds__(256) void kWordNegate(WordBits *__restrict__ wb, double *__restrict__ val, Frame f,
+                                                   uint32_t nw) {
+  const uint32_t lane = threadIdx.x & 63u;
+  forWords(
+      nw + 1, xcdOrder(blockIdx.x, gridDim.x), gridDim.x,
+      [&](uint32_t w) -> uint64_t {
+        const WordBits b = wb[w];
+        const uint64_t ok = w < nw ? validOf(f, w) : (f.base ? 1ull : 0ull);
+        if (!uniformWord(b, ok)) return 1ull;
+        wb[w].neg = ~b.neg & ok;
+        return 0ull;
+      },
+      [&](uint32_t w, uint64_t) {
+        const uint64_t ok = w < nw ? validOf(f, w) : 1ull;
+        double v = -val[(w << 6) | lane];
+        v = __builtin_amdgcn_inverse_ballot_w64(ok) ? v : POS;
+        putWord(wb, val, w, lane, v);
+      });
+}
+void launchWordNegate(hipStream_t s, const WordBufs &b, const Frame &f) {
+  const uint32_t nw = (uint32_t)f.nwords;
+  kWordNegate<<<wordGrid(nw + 1), TPB, 0, s>>>(b.wb, b.val, f, nw);
+}
+
+}  // namespace lsg

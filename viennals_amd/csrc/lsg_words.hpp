@@ -1,0 +1,810 @@
+// Word bands: the dense-frame form of a level-set band that the band
+// operations of a time step read and write.
+//
+// A word band holds, for every 64-point word of the frame (lsg_device.hpp:
+// Frame), which of its points are defined and the sign of every point
+// (WordBits), and one value slot per grid point, val[p].  A word whose points
+// are all undefined and of one sign is uniform: its slots hold nothing.  In
+// every other word all slots hold the points' values, NEG and POS among them,
+// so that an operation reads a whole word with one load per lane.  Word nwords
+// holds the grid-minimum entry of a band whose frame does not contain the grid
+// minimum, in its bit 0.  Two pages of 64 slots in front of the words, all POS
+// and all NEG, stand for the slots of uniform words.  Compared with the
+// canonical run list (values packed in entry order behind prefix counts) a
+// lookup needs no rank, so a band operation needs no scan: one kernel
+// evaluates a rule and writes the result.  The run starts of the canonical
+// list (every defined point, and every undefined point whose value differs
+// from the point before it) follow from WordBits alone.
+//
+// Everything here is host and device code: the CPU tests run it against the
+// run-list pipeline.
+#pragma once
+
+#include "lsg_items.hpp"
+
+namespace lsg {
+
+struct alignas(16) WordBits {
+  uint64_t def;  // defined points
+  uint64_t neg;  // points with a value below 0 (0 past the row's end)
+};
+LSG_HD inline bool uniformWord(const WordBits &b, uint64_t valid) { return !b.def && (!b.neg || b.neg == valid); }
+
+// Byte offset of a word's slots from the first page, and the pages of the
+// uniform words.  Offsets are 32-bit, which bounds the frame.
+constexpr uint32_t WORD_PAGES = 2, PAGE_POS = 0, PAGE_NEG = 512;
+LSG_HD inline uint32_t wordOffset(uint32_t w) { return (w + WORD_PAGES) << 9; }
+// Frames up to this size (2^29 points: 4 GiB of value slots) have word bands.
+constexpr int64_t WORD_BAND_MAX_WORDS = ((int64_t)1 << 23) - WORD_PAGES - 1;
+
+LSG_HD inline int wordLast(const Frame &f) { return (f.ext[0] - 1) >> 6; }
+LSG_HD inline int rowLastBit(const Frame &f) { return (f.ext[0] - 1) & 63; }
+// The points of word kw of a row (the last word of a row may be partial).
+LSG_HD inline uint64_t wordValid(const Frame &f, int kw) {
+  if (kw != wordLast(f)) return ~0ull;
+  const int nb = rowLastBit(f) + 1;
+  return nb < 64 ? (~0ull >> (64 - nb)) : ~0ull;
+}
+
+// One grid point of a word band, or (bit < 0) the point of the same bit in
+// another word.
+struct WordRef {
+  uint32_t w;
+  int bit;
+};
+
+// The frame point before the start of row `row` (rows counted over y and z):
+// the last point of the row before it, or the grid-minimum entry.
+LSG_HD inline WordRef beforeRow(const Frame &f, int32_t row) {
+  if (row <= 0) return WordRef{(uint32_t)f.nwords, 0};
+  return WordRef{(uint32_t)((row - 1) * f.wpr + wordLast(f)), rowLastBit(f)};
+}
+
+// An absolute, in-grid point; outside the frame the frame point before it in
+// HRLE order.
+LSG_HD inline WordRef frameRef(const Frame &f, int32_t x, int32_t y, int32_t z) {
+  const int64_t xr = (int64_t)x - f.o[0];
+  const int64_t yr = (int64_t)y - f.o[1];
+  const int64_t zr = (int64_t)z - f.o[2];
+  if (zr < 0) return beforeRow(f, 0);
+  if (zr >= f.ext[2]) return beforeRow(f, f.ext[1] * f.ext[2]);
+  if (yr < 0) return beforeRow(f, (int32_t)zr * f.ext[1]);
+  if (yr >= f.ext[1]) return beforeRow(f, (int32_t)(zr + 1) * f.ext[1]);
+  const int32_t row = (int32_t)zr * f.ext[1] + (int32_t)yr;
+  if (xr < 0) return beforeRow(f, row);
+  if (xr >= f.ext[0]) return beforeRow(f, row + 1);
+  return WordRef{(uint32_t)(row * f.wpr) + (uint32_t)(xr >> 6), (int)(xr & 63)};
+}
+
+// A frame with the boundary mapping of a single star step, which only
+// matters at the frame's faces: first[d] is where the step -1 from frame
+// coordinate 0 lands, last[d] the step +1 from ext[d] - 1 (-1 and ext[d]:
+// outside the frame).
+struct WordFrame {
+  Frame f;
+  int32_t first[3], last[3];
+  int bounded0, periodic0;
+  // the star of the grid-minimum entry: itself, then +1 and -1 along each
+  // axis (word | bit << 24)
+  uint32_t gmin[7];
+  LSG_HD void init(const Frame &f_, const GridInfo &g) {
+    f = f_;
+    for (int d = 0; d < 3; ++d) {
+      first[d] = -1;
+      last[d] = f.ext[d];
+      if (d >= g.D) continue;
+      const int32_t a = g.map(d, (int64_t)f.o[d] - 1), b = g.map(d, (int64_t)f.o[d] + f.ext[d]);
+      if (a >= f.o[d] && a - f.o[d] < f.ext[d]) first[d] = a - f.o[d];
+      if (b >= f.o[d] && b - f.o[d] < f.ext[d]) last[d] = b - f.o[d];
+    }
+    bounded0 = g.bounded(0) ? 1 : 0;
+    periodic0 = g.bc[0] == PERIODIC ? 1 : 0;
+    for (int k = 0; k < 7; ++k) {
+      int32_t c[3] = {g.lo[0], g.lo[1], g.lo[2]};
+      const int d = (k - 1) >> 1;
+      if (k > 0 && d < g.D) c[d] = g.map(d, (int64_t)c[d] + ((k & 1) ? 1 : -1));
+      const WordRef r = frameRef(f, c[0], c[1], c[2]);
+      gmin[k] = r.w | ((uint32_t)r.bit << 24);
+    }
+  }
+  // Frame coordinate a step s away along axis d (-1 or ext[d]: outside).
+  LSG_HD int32_t step(int d, int32_t x, int s) const {
+    if (s < 0) return x > 0 ? x - 1 : first[d];
+    return x < f.ext[d] - 1 ? x + 1 : last[d];
+  }
+};
+
+// The star neighbour of the points of word w = (kw, yr, zr) one step s along
+// axis d >= 1: the word a step away, or, when the step leaves the frame, the
+// one point all of them see (the frame point before that place in HRLE
+// order: BandView::locate's rule).
+LSG_HD inline WordRef stepRef(const WordFrame &F, uint32_t w, int32_t yr, int32_t zr, int d, int s) {
+  const Frame &f = F.f;
+  const int32_t here = d == 1 ? yr : zr, rr = F.step(d, here, s);
+  if (rr >= 0 && rr < f.ext[d]) {
+    const int32_t stride = d == 1 ? f.wpr : f.wpr * f.ext[1];
+    return WordRef{w + (uint32_t)((rr - here) * stride), -1};
+  }
+  if (d == 1) return beforeRow(f, (rr < 0 ? zr : zr + 1) * f.ext[1]);
+  return beforeRow(f, rr < 0 ? 0 : f.ext[1] * f.ext[2]);
+}
+
+// The x neighbour of the first (s = -1) or last (s = +1) point of word w =
+// (kw, row).
+LSG_HD inline WordRef edgeRef(const WordFrame &F, uint32_t w, int kw, int32_t row, int s) {
+  const Frame &f = F.f;
+  if (s < 0 && kw > 0) return WordRef{w - 1u, 63};
+  if (s > 0 && kw < wordLast(f)) return WordRef{w + 1u, 0};
+  const int32_t rr = s < 0 ? F.first[0] : F.last[0];
+  if (rr < 0) return beforeRow(f, row);
+  if (rr >= f.ext[0]) return beforeRow(f, row + 1);
+  return WordRef{w - (uint32_t)kw + (uint32_t)(rr >> 6), (int)(rr & 63)};
+}
+
+// Lookups of a word band, with BandView's interface (the schemes of
+// lsg_items.hpp take either).
+struct WordView {
+  const WordBits *wb;  // nwords + 1
+  const double *val;   // 64 (nwords + 1), the pages before them
+  Frame f;
+  GridInfo g;
+
+  LSG_HD void coords(uint32_t p, int32_t c[3]) const {
+    int32_t xr, yr, zr;
+    f.decode(p, xr, yr, zr);
+    c[0] = xr + f.o[0];
+    c[1] = yr + f.o[1];
+    c[2] = zr + f.o[2];
+  }
+  LSG_HD BandView::Loc locate(int32_t x, int32_t y, int32_t z) const {
+    const WordRef r = frameRef(f, x, y, z);
+    BandView::Loc l;
+    l.w = r.w;
+    l.bt = (uint32_t)r.bit;
+    l.inside = true;
+    return l;
+  }
+  // Values at N located points.  The slots are read beside the words, not
+  // after them (every point has one; the stencils of the schemes lie in the
+  // band, so nearly all are defined), and the signs only where some point is
+  // undefined.
+  template <int N> LSG_HD void values(const BandView::Loc *l, double *out) const {
+    uint64_t q[N];
+    LSG_UNROLL
+    for (int k = 0; k < N; ++k) {
+      q[k] = wb[l[k].w].def;
+      out[k] = val[((size_t)l[k].w << 6) | l[k].bt];
+    }
+    uint64_t all = 1ull;
+    LSG_UNROLL
+    for (int k = 0; k < N; ++k) {
+      q[k] >>= l[k].bt;
+      all &= q[k];
+    }
+    if (all & 1ull) return;
+    LSG_UNROLL
+    for (int k = 0; k < N; ++k)
+      if (!(q[k] & 1ull)) out[k] = ((wb[l[k].w].neg >> l[k].bt) & 1ull) ? NEG : POS;
+  }
+  LSG_HD double point(uint32_t w, int bit) const {
+    const WordBits q = wb[w];
+    if ((q.def >> bit) & 1ull) return val[((size_t)w << 6) | (uint32_t)bit];
+    return ((q.neg >> bit) & 1ull) ? NEG : POS;
+  }
+  LSG_HD double value(int32_t x, int32_t y, int32_t z) const {
+    const BandView::Loc l = locate(x, y, z);
+    return point(l.w, (int)l.bt);
+  }
+};
+
+// ------------------------------------------------------------ run starts ----
+
+// def / neg of the point before word w in HRLE order (for the first word the
+// grid-minimum entry, or "defined" when the word holds the grid minimum
+// itself: its entry always starts a run).
+struct WordCarry {
+  uint64_t def, neg;
+};
+LSG_HD inline WordCarry wordCarry(const WordBits &prev, int kw, const Frame &f) {
+  const int b = kw > 0 ? 63 : rowLastBit(f);
+  return WordCarry{(prev.def >> b) & 1ull, (prev.neg >> b) & 1ull};
+}
+LSG_HD inline WordCarry firstCarry(const WordBits *wb, const Frame &f) {
+  if (!f.base) return WordCarry{1ull, 0ull};
+  const WordBits m = wb[f.nwords];
+  return WordCarry{m.def & 1ull, m.neg & 1ull};
+}
+// Run starts of a word: its defined points, the undefined ones after a
+// defined point and those of another sign than the point before.
+LSG_HD inline uint64_t startBits(const WordBits &b, const WordCarry &c) {
+  return b.def | (b.def << 1) | c.def | (b.neg ^ ((b.neg << 1) | c.neg));
+}
+LSG_HD inline uint64_t startsOfWord(const WordBits *wb, const Frame &f, uint32_t w) {
+  int32_t kw, yr, zr;
+  f.wordRow(w, kw, yr, zr);
+  const WordCarry c = w > 0 ? wordCarry(wb[w - 1], kw, f) : firstCarry(wb, f);
+  return startBits(wb[w], c) & wordValid(f, kw);
+}
+LSG_HD inline uint64_t topStart(const WordBits &b) {  // whether bit 63 starts a run
+  return (b.def >> 63) | (b.def >> 62 & 1ull) | ((b.neg >> 63) ^ (b.neg >> 62 & 1ull));
+}
+
+// What the operations read around one word: its own bits, the words (or the
+// single points, WordRef) its points see a step away along y and z, and the
+// points below its first and above its last one along x.
+template <int D> struct WordSite {
+  int32_t kw, yr, zr;
+  WordBits self;
+  WordRef ref[2 * D - 2];   // [2 (d - 1)] a step +1 along axis d, [2 (d - 1) + 1] a step -1
+  WordBits bits[2 * D - 2];
+  WordBits prev, prevs[2 * D - 2];  // the words before (of the row before at a row's start)
+  WordBits rowPrev;                 // periodic x: the word before the row
+  WordRef below, above;
+  int belowDef, belowNeg, aboveDef, aboveNeg;
+};
+template <int D> LSG_HD inline void wordSite(const WordBits *wb, const WordFrame &F, uint32_t w, WordSite<D> &s) {
+  const Frame &f = F.f;
+  f.wordRow(w, s.kw, s.yr, s.zr);
+  s.self = wb[w];
+  s.prev = wb[w > 0 ? w - 1u : 0u];
+  if (F.periodic0) s.rowPrev = wb[w > (uint32_t)s.kw ? w - (uint32_t)s.kw - 1u : 0u];
+  LSG_UNROLL
+  for (int d = 1; d < D; ++d)
+    LSG_UNROLL
+    for (int k = 0; k < 2; ++k) {
+      const WordRef r = stepRef(F, w, s.yr, s.zr, d, k ? -1 : 1);
+      s.ref[2 * d - 2 + k] = r;
+      s.bits[2 * d - 2 + k] = wb[r.w];
+      s.prevs[2 * d - 2 + k] = wb[r.w > 0 ? r.w - 1u : 0u];
+    }
+  const int32_t row = s.zr * f.ext[1] + s.yr;
+  s.below = edgeRef(F, w, s.kw, row, -1);
+  s.above = edgeRef(F, w, s.kw, row, 1);
+  const WordBits m = wb[s.below.w], p = wb[s.above.w];
+  s.belowDef = (int)(m.def >> s.below.bit & 1ull);
+  s.belowNeg = (int)(m.neg >> s.below.bit & 1ull);
+  s.aboveDef = (int)(p.def >> s.above.bit & 1ull);
+  s.aboveNeg = (int)(p.neg >> s.above.bit & 1ull);
+}
+
+// Whether every point that starPoints looks at is undefined and of one sign:
+// the word then has no point to evaluate and no conflict.
+template <int D> LSG_HD inline bool quietSite(const WordFrame &F, const WordSite<D> &s) {
+  const uint64_t valid = wordValid(F.f, s.kw), neg = (s.self.neg & 1ull) ? valid : 0ull;
+  const int last = s.kw > 0 ? 63 : rowLastBit(F.f);
+  const int sign = (int)(s.self.neg & 1ull);
+  if (s.kw == 0 && s.yr == 0 && s.zr == 0) return false;  // the carry is the grid-minimum entry's
+  uint64_t any = s.self.def | (s.self.neg ^ neg) | (s.prev.def >> last & 1ull) | ((s.prev.neg >> last & 1ull) ^ (uint64_t)sign);
+  if (s.kw > 0) any |= (s.prev.def >> 62 & 1ull) | ((s.prev.neg >> 62 & 1ull) ^ (uint64_t)sign);
+  any |= (uint64_t)(s.belowDef | s.aboveDef | (s.belowNeg ^ sign) | (s.aboveNeg ^ sign));
+  if (F.periodic0) {  // the row's first point, which the last one sees
+    const int lb = rowLastBit(F.f);
+    any |= (s.rowPrev.def >> lb & 1ull) | ((s.rowPrev.neg >> lb & 1ull) ^ (uint64_t)sign);
+    if (s.yr == 0 && s.zr == 0) any |= 1ull;
+  }
+  LSG_UNROLL
+  for (int k = 0; k < 2 * D - 2; ++k) {
+    const WordBits Q = s.bits[k], Qp = s.prevs[k];
+    if (s.ref[k].bit >= 0) any |= (Q.def >> s.ref[k].bit & 1ull) | ((Q.neg >> s.ref[k].bit & 1ull) ^ (uint64_t)sign);
+    else any |= Q.def | (Q.neg ^ neg) | (Qp.def >> last & 1ull) | ((Qp.neg >> last & 1ull) ^ (uint64_t)sign);
+    if (s.ref[k].w == 0) any |= 1ull;
+  }
+  return any == 0ull;
+}
+
+// Points of word w at which a star operation has to be evaluated: those whose
+// boundary-mapped star holds a run start.  Every other point is undefined and
+// keeps its value.
+//
+// The run-list pipeline (candStarWord) visits more points: the successors of
+// these and the first points of rows with a bounded x.  Their stars hold
+// undefined values only, so every rule returns the point's own value, except
+// the Expand rule where an undefined neighbour has the other sign: it then
+// changes the point, and in a run list all points after it up to the next
+// visited one.  Such fields (regions of opposite sign that touch without a
+// defined point) are not distance fields and have no word band counterpart:
+// `conflict` reports them, and the caller runs the operation on run lists.
+template <int D, bool CHECK>
+LSG_HD inline uint64_t starPoints(const WordBits *wb, const WordFrame &F, uint32_t w, const WordSite<D> &s,
+                                  bool &conflict) {
+  const Frame &f = F.f;
+  const int kw = s.kw, wl = wordLast(f), lb = rowLastBit(f);
+  const WordBits B = s.self;
+  const WordBits P = s.prev;
+  const WordCarry carry = w > 0 ? wordCarry(P, kw, f) : firstCarry(wb, f);
+  const uint64_t valid = wordValid(f, kw);
+  const uint64_t S = startBits(B, carry) & valid;
+  uint64_t dil = S | (S << 1) | (S >> 1);
+  uint64_t prevTop = 0, mixed = 0;
+  if (kw > 0) {
+    const uint64_t s63 = topStart(P);
+    dil |= s63;
+    if (CHECK)
+      prevTop = s63 | (P.def >> 62 & 1ull) | (P.def >> 61 & 1ull) | ((P.neg >> 62 & 1ull) ^ (P.neg >> 61 & 1ull)) |
+                (S & 1ull);
+  }
+  if (kw < wl)  // the next word's first point
+    dil |= ((uint64_t)s.aboveDef | (B.def >> 63) | ((uint64_t)s.aboveNeg ^ (B.neg >> 63))) << 63;
+  if (F.periodic0) {
+    if (kw == wl) {  // the last point's +x neighbour is the row's first
+      const uint32_t w0 = w - (uint32_t)kw;
+      const WordCarry c0 = w0 > 0 ? wordCarry(s.rowPrev, 0, f) : firstCarry(wb, f);
+      if (startBits(wb[w0], c0) & 1ull) dil |= 1ull << lb;
+      if ((uint64_t)s.aboveNeg != (B.neg >> lb & 1ull)) mixed |= 1ull << lb;
+    }
+    if (kw == 0) {  // the first point's -x neighbour is the row's last
+      dil |= (uint64_t)s.belowDef;
+      mixed |= (uint64_t)s.belowNeg ^ (B.neg & 1ull);
+    }
+  }
+  LSG_UNROLL
+  for (int k = 0; k < 2 * D - 2; ++k) {
+    const WordRef r = s.ref[k];
+    const WordBits Q = s.bits[k];
+    if (r.bit >= 0) {  // one point outside the frame's rows
+      if (CHECK) mixed |= (Q.def >> r.bit & 1ull) ? ~0ull : (B.neg ^ ((Q.neg >> r.bit & 1ull) ? ~0ull : 0ull));
+      continue;
+    }
+    const WordBits Qp = s.prevs[k];
+    const WordCarry qc = r.w > 0 ? wordCarry(Qp, kw, f) : firstCarry(wb, f);
+    dil |= startBits(Q, qc) & valid;
+    mixed |= B.neg ^ Q.neg;
+    if (CHECK && kw > 0) prevTop |= topStart(Qp);
+  }
+  dil &= valid;
+  if (CHECK) {
+    const uint64_t succ = (dil << 1) | prevTop | ((F.bounded0 && kw == 0) ? 1ull : 0ull);
+    if (succ & ~dil & mixed & valid) conflict = true;
+  }
+  return dil;
+}
+
+// Sign word of a boolean of two words without defined points (ruleBoolean on
+// undefined values).
+LSG_HD inline uint64_t boolNeg(int kind, uint64_t a, uint64_t b) {
+  if (kind == B_INTERSECT) return a & b;
+  if (kind == B_UNION) return a | b;
+  if (kind == B_RELCOMP) return a & ~b;
+  return a;  // combine: the first band's undefined value
+}
+
+// Word of a canonical run list: def / neg from the start bits and the
+// entries' values.  rank0 = entries before the word; every run start is
+// defined or undefined by its value, and an undefined point between starts
+// carries the value of the last entry at or before it.
+LSG_HD inline double runValueAt(const double *val, uint64_t starts, uint32_t rank0, int bit) {
+  const uint64_t upto = starts & (bit == 63 ? ~0ull : ((2ull << bit) - 1ull));
+  const uint32_t r = rank0 + (uint32_t)__builtin_popcountll(upto);
+  return val[r > 0 ? r - 1 : 0];
+}
+
+// ------------------------------------------------------------ operations ----
+
+enum WordOp : int {
+  W_EXPAND = 0,       // one Expand cycle (limit a, totalLimit b)
+  W_REBUILD = 1,      // Advect::rebuildLS (cutoff a)
+  W_UPD_REBUILD = 2,  // updateLevelSet, then rebuildLS (cutoff a)
+  W_REDUCE = 3,       // Reduce (value limit a)
+  W_PRUNE = 4,
+  W_PRUNE_RSZ = 5     // Prune with removeStrayZeros
+};
+
+// A star operation's rule from the star's values (for W_UPD_REBUILD the
+// updated values).
+template <int D, int OP> LSG_HD inline double wordRule(double c, const double *nb, double a, double b) {
+  if (OP == W_EXPAND) {  // ruleExpand from the star's extremes (ruleExpandMinMax)
+    double lo = POS, hi = NEG;
+    LSG_UNROLL
+    for (int k = 0; k < 2 * D; ++k) {
+      lo = fmin(lo, nb[k]);
+      hi = fmax(hi, nb[k]);
+    }
+    return ruleExpandMinMax(c, lo, hi, a, b);
+  }
+  if (OP == W_REBUILD || OP == W_UPD_REBUILD) return ruleRebuild<D>(c, nb, a);
+  if (OP == W_REDUCE) return ruleReduce(c, a);
+  return rulePrune<D>(c, nb, OP == W_PRUNE_RSZ);
+}
+
+// The rule at one absolute grid point through general lookups (what the word
+// kernels are tested against).
+template <int D, int OP>
+LSG_HD inline double wordRuleAt(const WordView &v, const int32_t c[3], const double *rates, double dt, double a,
+                                double b) {
+  double u[2 * D + 1];
+  for (int k = 0; k < 2 * D + 1; ++k) {
+    int32_t p[3] = {c[0], c[1], c[2]};
+    const int d = k % D;
+    if (k < 2 * D) p[d] = v.g.map(d, (int64_t)c[d] + (k < D ? 1 : -1));
+    const WordRef r = frameRef(v.f, p[0], p[1], p[2]);
+    u[k] = v.point(r.w, r.bit);
+    if (OP == W_UPD_REBUILD) u[k] = ruleUpdate(u[k], dt, isUndef(u[k]) ? 0. : rates[((size_t)r.w << 6) | (uint32_t)r.bit]);
+  }
+  return wordRule<D, OP>(u[2 * D], u, a, b);
+}
+// The rule at the grid-minimum entry; `old` its value before.
+template <int D, int OP>
+LSG_HD inline double wordRuleMin(const WordFrame &F, const WordBits *wb, const double *val, const double *rates,
+                                 double dt, double a, double b, double &old) {
+  double u[2 * D + 1];
+  LSG_UNROLL
+  for (int k = 0; k < 2 * D + 1; ++k) {
+    const uint32_t w = F.gmin[k] & 0xFFFFFFu, bit = F.gmin[k] >> 24;
+    const WordBits q = wb[w];
+    const bool def = (q.def >> bit) & 1ull;
+    const size_t slot = ((size_t)w << 6) | bit;
+    double x = val[slot];
+    x = def ? x : (((q.neg >> bit) & 1ull) ? NEG : POS);
+    if (k == 0) old = x;
+    if (OP == W_UPD_REBUILD) x = ruleUpdate(x, dt, rates[slot]);
+    u[k == 0 ? 2 * D : ((k - 1) >> 1) + ((k & 1) ? 0 : D)] = x;
+  }
+  return wordRule<D, OP>(u[2 * D], u, a, b);
+}
+
+// ------------------------------------------------------------- schemes ----
+// The one-dimensional schemes of lsg_items.hpp (same expressions, same order
+// of operations) with one pass of a rolled loop per axis: the code of a
+// kernel stays small enough for the instruction cache, which a workgroup
+// that evaluates one or two waves of points otherwise fills from memory, and
+// one axis' values are in flight at a time.
+
+// Values at distance K0 .. K along axis d of point p (frame coordinates r,
+// absolute c): st[K + k] = phi(c + k e_d).  Every point is a slot at a fixed
+// offset where the axis is bounded and longer than K, or p is K cells inside
+// the frame; elsewhere, and where one of them is undefined, each is looked up
+// on its own.
+template <int K0, int K>
+LSG_HD inline void axisValues(const WordView &v, uint32_t p, const int32_t r[3], int d, double *st) {
+  const int32_t x = d == 0 ? r[0] : (d == 1 ? r[1] : r[2]);
+  const int32_t ext = v.f.ext[d];
+  const int32_t stride = d == 0 ? 1 : (d == 1 ? (int32_t)v.f.rowBits() : v.f.ext[1] * (int32_t)v.f.rowBits());
+  const bool inner = x >= K && x + K < ext;
+  const bool per = v.g.bc[d] == PERIODIC;
+  bool ok = inner || (v.g.bounded(d) && ext > K);
+  uint64_t all = 1ull;
+  LSG_UNROLL
+  for (int k = -K; k <= K; ++k) {
+    if (k > -K0 && k < K0) continue;
+    int32_t y = x + k;
+    if (k < 0) y = y >= 0 ? y : (per ? y + ext : -y);
+    else y = y < ext ? y : (per ? y - ext : 2 * (ext - 1) - y);
+    const uint32_t q = ok ? p + (uint32_t)((y - x) * stride) : p;
+    all &= v.wb[q >> 6].def >> (q & 63u);
+    st[K + k] = v.val[q];
+  }
+  if (ok && (all & 1ull)) return;
+#if defined(__clang__)
+#pragma unroll 1
+#endif
+  for (int k = -K; k <= K; ++k) {
+    if (k > -K0 && k < K0) continue;
+    int32_t c[3] = {r[0] + v.f.o[0], r[1] + v.f.o[1], r[2] + v.f.o[2]};
+    const int32_t m = v.g.map(d, (int64_t)x + v.f.o[d] + k);
+    const WordRef o = frameRef(v.f, d == 0 ? m : c[0], d == 1 ? m : c[1], d == 2 ? m : c[2]);
+    const double u = v.point(o.w, o.bit);
+    LSG_UNROLL
+    for (int j = 0; j < 2 * K + 1; ++j) st[j] = j == K + k ? u : st[j];
+  }
+}
+
+// One double per axis with an index that is not a constant.
+struct Axes {
+  double v[3] = {0., 0., 0.};
+  LSG_HD void set(int d, double x) {
+    v[0] = d == 0 ? x : v[0];
+    v[1] = d == 1 ? x : v[1];
+    v[2] = d == 2 ? x : v[2];
+  }
+};
+
+// schemeWENO
+template <int D, int ORDER>
+LSG_HD inline RateOut wordWENO(const WordView &b, uint32_t p, const int32_t r[3], double phi0, bool calcNormals,
+                               const Vel &vel) {
+  constexpr int R = (ORDER + 1) / 2;
+  double gradPosTotal = 0, gradNegTotal = 0, denominator = 0;
+  Axes gm, gp, n;
+#if defined(__clang__)
+#pragma unroll 1
+#endif
+  for (int d = 0; d < D; ++d) {
+    double st[2 * R + 1];
+    axisValues<1, R>(b, p, r, d, st);
+    st[R] = phi0;
+    const double cd = st[R + 1] - st[R - 1];
+    double m, q;
+    if (ORDER == 3) {
+      m = weno3(st, b.g.dx, false);
+      q = weno3(st, b.g.dx, true);
+    } else {
+      m = weno5(st, b.g.dx, false);
+      q = weno5(st, b.g.dx, true);
+    }
+    gradPosTotal += pow2(dmaxs(m, 0.0)) + pow2(dmins(q, 0.0));
+    gradNegTotal += pow2(dmins(m, 0.0)) + pow2(dmaxs(q, 0.0));
+    gm.set(d, m);
+    gp.set(d, q);
+    if (calcNormals) {
+      n.set(d, cd);
+      denominator += cd * cd;
+    }
+  }
+  if (calcNormals && denominator > 0) {
+    denominator = 1. / sqrt(denominator);
+    LSG_UNROLL
+    for (int i = 0; i < D; ++i) n.v[i] *= denominator;
+  }
+  double vel_grad = 0.;
+  const double sv = vel.scalar(n.v);
+  if (sv > 0) vel_grad += sqrt(gradPosTotal) * sv;
+  else vel_grad += sqrt(gradNegTotal) * sv;
+  LSG_UNROLL
+  for (int w = 0; w < D; w++) {
+    if (vel.vec[w] > 0.) vel_grad += vel.vec[w] * gm.v[w];
+    else vel_grad += vel.vec[w] * gp.v[w];
+  }
+  return {vel_grad, 0.};
+}
+
+// One-sided differences of every axis (gatherUpwind, upwindDiffs): pos[d] =
+// diffNeg, neg[d] = diffPos as the schemes name their gradients; `each(d,
+// diffPos, diffNeg, centred)` accumulates, centred = ((phi+ - phi0) + (phi0 -
+// phi-)) / 2.
+template <int D, class Each>
+LSG_HD inline void wordUpwind(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order, Axes &pos,
+                              Axes &neg, Each each) {
+#if defined(__clang__)
+#pragma unroll 1
+#endif
+  for (int d = 0; d < D; ++d) {
+    double st[5], s1[3];
+    axisValues<1, 1>(b, p, r, d, s1);
+    st[0] = st[4] = 0.;
+    if (order == 2) axisValues<2, 2>(b, p, r, d, st);
+    st[1] = s1[0];
+    st[3] = s1[2];
+    double diffPos, diffNeg;
+    upwindDiffs(st, b.g.dx, order, phi0, diffPos, diffNeg);
+    pos.set(d, diffNeg);
+    neg.set(d, diffPos);
+    each(d, diffPos, diffNeg, ((st[3] - phi0) + (phi0 - st[1])) * 0.5);
+  }
+}
+
+// schemeEO
+template <int D>
+LSG_HD inline RateOut wordEO(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
+                             bool calcNormals, const Vel &vel) {
+  Axes pos, neg, n;
+  double gradPosTotal = 0, gradNegTotal = 0, denominator = 0;
+  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double centred) {
+    gradPosTotal += pow2(dmaxs(diffNeg, 0.0)) + pow2(dmins(diffPos, 0.0));
+    gradNegTotal += pow2(dmins(diffNeg, 0.0)) + pow2(dmaxs(diffPos, 0.0));
+    if (calcNormals) {
+      n.set(d, centred);
+      denominator += centred * centred;
+    }
+  });
+  if (calcNormals) {
+    denominator = 1. / sqrt(denominator);
+    LSG_UNROLL
+    for (int i = 0; i < D; ++i) n.v[i] *= denominator;
+  }
+  double vel_grad = 0.;
+  const double sv = vel.scalar(n.v);
+  if (sv > 0) vel_grad += sqrt(gradPosTotal) * sv;
+  else vel_grad += sqrt(gradNegTotal) * sv;
+  LSG_UNROLL
+  for (int w = 0; w < D; w++) {
+    if (vel.vec[w] > 0.) vel_grad += vel.vec[w] * pos.v[w];
+    else vel_grad += vel.vec[w] * neg.v[w];
+  }
+  return {vel_grad, 0.};
+}
+
+// schemeLF
+template <int D>
+LSG_HD inline RateOut wordLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
+                             bool calcNormals, const Vel &vel, double alphaFactor, const double *alphas) {
+  Axes pos, neg, n;
+  double grad = 0., dissipation = 0., modulus = 0.;
+  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double) {
+    const double m = (diffNeg + diffPos) * 0.5;
+    if (calcNormals) {
+      n.set(d, m);
+      modulus += m * m;
+    }
+    grad += pow2(m);
+    const double alpha = d == 0 ? alphas[0] : (d == 1 ? alphas[1] : alphas[2]);
+    dissipation += alphaFactor * alpha * (diffPos - diffNeg) * 0.5;
+  });
+  if (calcNormals) {
+    modulus = 1. / sqrt(modulus);
+    LSG_UNROLL
+    for (int i = 0; i < D; ++i) n.v[i] *= modulus;
+  }
+  const double sv = vel.scalar(n.v);
+  double totalGrad = 0.;
+  if (sv != 0.) totalGrad = sv * sqrt(grad);
+  LSG_UNROLL
+  for (int w = 0; w < D; w++) {
+    if (vel.vec[w] > 0.) totalGrad += vel.vec[w] * pos.v[w];
+    else totalGrad += vel.vec[w] * neg.v[w];
+  }
+  return {totalGrad, (totalGrad != 0.) ? dissipation : 0};
+}
+
+// The gradient part that schemeLLLF and schemeLLF share: the total gradient
+// and the normalised centred gradient.
+template <int D>
+LSG_HD inline double wordLocalGradient(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
+                                       const Vel &vel, Axes &pos, Axes &neg, Axes &n, double &sv) {
+  double grad = 0., modulus = 0.;
+  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double) {
+    const double m = (diffNeg + diffPos) * 0.5;
+    n.set(d, m);
+    modulus += m * m;
+    grad += pow2(m);
+  });
+  modulus = 1. / sqrt(modulus);
+  LSG_UNROLL
+  for (int i = 0; i < D; ++i) n.v[i] *= modulus;
+  sv = vel.scalar(n.v);
+  double totalGrad = 0.;
+  if (sv != 0.) totalGrad = sv * sqrt(grad);
+  LSG_UNROLL
+  for (int w = 0; w < D; w++) {
+    if (vel.vec[w] > 0.) totalGrad += vel.vec[w] * pos.v[w];
+    else totalGrad += vel.vec[w] * neg.v[w];
+  }
+  return totalGrad;
+}
+
+// schemeLLLF
+template <int D>
+LSG_HD inline RateOut wordLLLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
+                               const Vel &vel, double alphaFactor, double *alphaAcc) {
+  Axes pos, neg, n;
+  double sv;
+  const double totalGrad = wordLocalGradient<D>(b, p, r, phi0, order, vel, pos, neg, n, sv);
+  if (totalGrad == 0.) return {0., 0.};
+  double dissipation = 0.;
+  LSG_UNROLL
+  for (int i = 0; i < D; ++i) {
+    const double alpha = fabs((sv + vel.vec[i]) * n.v[i]);
+    alphaAcc[i] = dmaxs(alphaAcc[i], alpha);
+    dissipation += alphaFactor * alpha * (neg.v[i] - pos.v[i]) * 0.5;
+  }
+  return {totalGrad, dissipation};
+}
+
+// Alphas of the local Lax-Friedrichs box at one grid point from its star
+// (llfBoxNormalFrom and the box loop of schemeLLF): |(scalar + vector_k) n_k|.
+// Division by a grid delta of 1 is the identity.
+template <int D>
+LSG_HD inline void boxAlphas(const double *bv, double dx, const Vel &vel, double *t) {
+  double n[3] = {0., 0., 0.};
+  double nm = 0.;
+  const double center = bv[2 * D];
+  LSG_UNROLL
+  for (int dir = 0; dir < D; ++dir) {
+    double dP = bv[dir] - center, dN = center - bv[D + dir];
+    if (dx != 1.) {
+      dP = dP / dx;
+      dN = dN / dx;
+    }
+    n[dir] = (dP + dN) * 0.5;
+    nm += n[dir] * n[dir];
+  }
+  nm = 1. / sqrt(nm);
+  LSG_UNROLL
+  for (int dir = 0; dir < D; ++dir) n[dir] *= nm;
+  const double sv = vel.scalar(n);
+  LSG_UNROLL
+  for (int dir = 0; dir < D; ++dir) t[dir] = fabs((sv + vel.vec[dir]) * n[dir]);
+}
+// Whether the box alphas of a point serve every active point around it.  A
+// box point beyond a mirror boundary has the mirrored normal of the point it
+// maps to: all its products keep their magnitude unless the built-in speed
+// depends on the sign of that component.  The axes must be longer than the
+// box' stencil, and an open axis must not end inside the frame's reach.
+LSG_HD inline bool boxAlphasShared(const GridInfo &g, const Frame &f, const Vel &vel) {
+  for (int d = 0; d < g.D; ++d) {
+    if (g.bc[d] == REFLECTIVE && vel.kind == 1 && d == vel.dir) return false;
+    if (g.bounded(d) ? f.ext[d] < 3 : (g.bc[d] != INFINITE || f.o[d] == g.lo[d] || f.o[d] + f.ext[d] - 1 == g.hi[d]))
+      return false;
+  }
+  return true;
+}
+// Value index of component k of the box alphas at frame position p.
+template <int D> LSG_HD inline size_t boxSlot(uint32_t p, int k) {
+  return ((size_t)(p >> 6) * D + (size_t)k) * 64 + (p & 63u);
+}
+
+// schemeLLF with the box alphas of the band's points at hand; `outside` is
+// set where a box point lies outside the frame (nothing is read there).
+template <int D>
+LSG_HD inline RateOut wordLLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
+                              const Vel &vel, double alphaFactor, double *alphaAcc, const double *box, bool &outside) {
+  Axes pos, neg, n;
+  double sv;
+  const double totalGrad = wordLocalGradient<D>(b, p, r, phi0, order, vel, pos, neg, n, sv);
+  if (totalGrad == 0.) return {0., 0.};
+  // slot offsets of the steps -1, 0, +1 along each axis
+  int32_t off[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
+  LSG_UNROLL
+  for (int d = 0; d < D; ++d) {
+    const int32_t ext = b.f.ext[d], x = r[d];
+    const int32_t stride = d == 0 ? 1 : (d == 1 ? (int32_t)b.f.rowBits() : b.f.ext[1] * (int32_t)b.f.rowBits());
+    int32_t lo = x - 1, hi = x + 1;
+    if (b.g.bounded(d)) {
+      const bool per = b.g.bc[d] == PERIODIC;
+      if (lo < 0) lo = per ? lo + ext : -lo;
+      if (hi >= ext) hi = per ? hi - ext : 2 * (ext - 1) - hi;
+    } else if (lo < 1 || hi >= ext - 1) {
+      outside = true;
+      return {0., 0.};
+    }
+    off[d][0] = (lo - x) * stride;
+    off[d][2] = (hi - x) * stride;
+  }
+  double alpha[D];
+  LSG_UNROLL
+  for (int i = 0; i < D; ++i) alpha[i] = 0;
+#if defined(__clang__)
+#pragma unroll 1
+#endif
+  for (int q = 0; q < (D == 3 ? 9 : 3); ++q) {
+    const int qy = D == 3 ? q % 3 : q, qz = D == 3 ? q / 3 : 1;
+    int32_t o = qy == 0 ? off[1][0] : (qy == 1 ? 0 : off[1][2]);
+    if (D == 3) o += qz == 0 ? off[2][0] : (qz == 1 ? 0 : off[2][2]);
+    double t[3 * D];
+    LSG_UNROLL
+    for (int x = 0; x < 3; ++x)
+      LSG_UNROLL
+      for (int k = 0; k < D; ++k) t[x * D + k] = box[boxSlot<D>(p + (uint32_t)(o + off[0][x]), k)];
+    LSG_UNROLL
+    for (int x = 0; x < 3; ++x)
+      LSG_UNROLL
+      for (int k = 0; k < D; ++k) alpha[k] = fmax(alpha[k], t[x * D + k]);
+  }
+  double dissipation = 0.;
+  LSG_UNROLL
+  for (int i = 0; i < D; ++i) {
+    alphaAcc[i] = fmax(alphaAcc[i], alpha[i]);
+    dissipation += alphaFactor * alpha[i] * (neg.v[i] - pos.v[i]) * 0.5;
+  }
+  return {totalGrad, dissipation};
+}
+
+// The local Lax-Friedrichs scheme with shared box alphas (a scheme id of the
+// word kernels beside SchemeId's).
+constexpr int S_LLF_BOX = 16;
+
+// ratePoint for an active point of a word band.
+template <int D, int SCHEME>
+LSG_HD inline double wordRatePoint(const WordView &v, uint32_t p, const RateParams &rp, const Vel &vel,
+                                   const double *globalAlphas, double *alphaAcc, double &velocity, bool &sllfUsed,
+                                   const double *box = nullptr, bool *outside = nullptr) {
+  int32_t r[3];
+  v.f.decode(p, r[0], r[1], r[2]);
+  const double phi0 = v.val[p];
+  RateOut o;
+  if (SCHEME == S_EO) o = wordEO<D>(v, p, r, phi0, rp.order, rp.calcNormals != 0, vel);
+  else if (SCHEME == S_WENO5) o = wordWENO<D, 5>(v, p, r, phi0, rp.calcNormals != 0, vel);
+  else if (SCHEME == S_WENO3) o = wordWENO<D, 3>(v, p, r, phi0, rp.calcNormals != 0, vel);
+  else if (SCHEME == S_LF) o = wordLF<D>(v, p, r, phi0, rp.order, rp.calcNormals != 0, vel, rp.alphaFactor, globalAlphas);
+  else if (SCHEME == S_LLLF) o = wordLLLF<D>(v, p, r, phi0, rp.order, vel, rp.alphaFactor, alphaAcc);
+  else if (SCHEME == S_LLF_BOX) o = wordLLF<D>(v, p, r, phi0, rp.order, vel, rp.alphaFactor, alphaAcc, box, *outside);
+  else {
+    const int32_t c[3] = {r[0] + v.f.o[0], r[1] + v.f.o[1], r[2] + v.f.o[2]};
+    return ratePoint<D, SCHEME>(v, c, phi0, rp, vel, globalAlphas, alphaAcc, velocity, nullptr, nullptr, &sllfUsed);
+  }
+  velocity = o.H - o.Dn;
+  double x = velocity;
+  if ((rp.checkDissipation && (o.H < 0 && x > 0)) || (o.H > 0 && x < 0)) x = 0;
+  return x;
+}
+
+}  // namespace lsg

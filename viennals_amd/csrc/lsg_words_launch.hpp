@@ -1,0 +1,81 @@
+// Host-visible launch interface of the word-band kernels (lsg_words.hip).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "lsg_kernels.hpp"
+#include "lsg_words.hpp"
+
+namespace lsg {
+
+struct WordBufs {
+  WordBits *wb = nullptr;  // nwords + 1
+  double *val = nullptr;   // 64 (nwords + 1), behind 64 WORD_PAGES slots of the same allocation
+};
+// Fills the pages of uniform words of a new allocation (`pages` its start).
+void launchWordPages(hipStream_t s, double *pages);
+
+// Device scalars of one step on word bands.  The maxima are spread over
+// STEP_SLOTS addresses (workgroup b adds to slot b % STEP_SLOTS); the kernel
+// that needs a stage's time step reduces them in every wave.
+constexpr int STEP_SLOTS = 64;
+constexpr int STEP_STAGES = 3;
+struct WordStep {
+  double maxTimeStep;
+  double dt[4];
+  uint32_t reframe;
+  uint32_t conflict;  // an Expand met a field word bands do not hold (starPoints); cleared by the host
+  unsigned long long active[STEP_STAGES][STEP_SLOTS];
+  // not read by the host
+  unsigned long long maxAbs[STEP_STAGES][STEP_SLOTS];
+  unsigned long long alpha[STEP_STAGES][3][STEP_SLOTS];
+  unsigned long long sllfKey[STEP_STAGES];  // SLLF: frame position + 1 of the last point that set its alphas
+  double starBytes[STEP_SLOTS];             // profiling: algorithmic bytes of the star operations / rate passes
+  double rateBytes[STEP_SLOTS];
+};
+
+struct WordOpArgs {
+  double a = 0, b = 0;  // the rule's limits
+  // W_UPD_REBUILD: the stage whose maxima give the time step
+  int stage = 0, useAlphas = 0;
+  double cfl = 0;
+  const double *maxDt = nullptr;
+  const double *rates = nullptr;
+  int slack = 0;       // > 0: flag WordStep::reframe when a defined point is closer than this to an open frame edge
+  int count = 0;       // profiling: add the algorithmic bytes to starBytes
+  uint64_t *act = nullptr;        // active points (|phi| <= 1/2) of the result, one word each
+  const uint64_t *inAct = nullptr;  // W_UPD_REBUILD: active points of the input
+  const double *begin = nullptr;  // the step's first operation: reset the scalars, take the bound from here
+};
+
+void launchWordBegin(hipStream_t s, WordStep *st, const double *maxDt);
+void launchWordStar(hipStream_t s, int D, int op, const WordBufs &in, const WordBufs &out, const Frame &f,
+                    const GridInfo &g, const WordOpArgs &a, WordStep *st);
+void launchWordBoolean(hipStream_t s, const WordBufs &A, const WordBufs &B, const WordBufs &out, const Frame &f,
+                       int kind, double wTarget, double wSource);
+void launchWordActive(hipStream_t s, const WordBufs &b, const Frame &f, uint64_t *act);
+// The passes over the active points of a band (act: their bits).
+// box: room for the local Lax-Friedrichs box alphas (64 D (nwords + 1)
+// doubles) where they can be shared (boxAlphasShared), else null.
+// LF global alphas of the stage (Advect::findGlobalAlphas).
+void launchWordAlphas(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
+                      const uint64_t *act, int stage, WordStep *st);
+void launchWordRates(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
+                     const uint64_t *act, double *rates, double *box, int stage, int count, WordStep *st,
+                     hipEvent_t e0 = nullptr,
+                     hipEvent_t e1 = nullptr, bool externalEvents = false);
+// Canonical run list <-> word band.
+void launchWordImport(hipStream_t s, const BandBufs &in, const WordBufs &out, const Frame &f);
+void launchWordExport(hipStream_t s, const WordBufs &in, BandBufs &out, const Frame &f, const GridInfo &g,
+                      uint32_t *partials, uint32_t *total);
+void launchWordCopy(hipStream_t s, const WordBufs &in, const WordBufs &out, const Frame &f);
+// The band of `in` (frame f) on another frame.
+void launchWordReframe(hipStream_t s, const WordBufs &in, const Frame &f, const GridInfo &g, const WordBufs &out,
+                       const Frame &fo);
+// Defined points (the grid-minimum entry included) and the bounding box of
+// the run starts inside the frame; *conflict takes WordStep::conflict.
+void launchWordStats(hipStream_t s, const WordBufs &b, const Frame &f, uint32_t *outCount, int32_t *bbox,
+                     const WordStep *st, uint32_t *conflict);
+void launchWordNegate(hipStream_t s, const WordBufs &b, const Frame &f);
+
+}  // namespace lsg
