@@ -70,6 +70,31 @@ def test_training_gradient_matches_oracle():
         assert np.linalg.norm(g - gref) <= 1e-3 * np.linalg.norm(gref)
 
 
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 1024 * 32 + 5])
+def test_training_gradient_at_tile_edges(n):
+    """One sample, a tile of 32 with one missing and one over, and more tiles
+    than workgroups: loss and gradient against the oracle, one optimiser step
+    against Adam on that gradient (few float32 operations per parameter)."""
+    from viennals_amd.learned import Trainer
+    P = rand_params(41, 0.3)
+    X, T = teacher_samples(42, n, rand_params(43, 0.5))
+    tr = Trainer(P)
+    tr.set_samples(X, T)
+    loss, g = tr.loss_grad()
+    lref, gref = po.mlp_loss_grad(P, X, T, emulate=True)
+    # as above; a single sample has no other to average its roundings with:
+    # a flipped bf16 rounding of an activation moves it by up to 2^-8
+    few = 1.0 if n >= 31 else 4.0
+    assert abs(loss - lref) <= few * 2e-3 * abs(lref), (loss, lref)
+    assert np.linalg.norm(g - gref) <= few * 2e-3 * np.linalg.norm(gref)
+    tr.train(1, n, 1e-2)
+    m, v = 0.1 * g.astype(np.float64), 0.001 * g.astype(np.float64) ** 2
+    want = P - 1e-2 * (m / 0.1) / (np.sqrt(v / 0.001) + 1e-8)
+    # 1 - 0.999f holds 0.001 to 6e-5 and the root halves that; the rest is a
+    # handful of roundings of 6e-8; the step has length <= 1e-2
+    assert np.abs(tr.params() - want).max() <= 1e-2 * 1e-4 + 2e-7 * np.abs(P).max()
+
+
 def test_training_reduces_loss_on_teacher_task():
     from viennals_amd.learned import Trainer, init_params
     teacher = rand_params(31, 0.4)

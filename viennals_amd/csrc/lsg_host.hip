@@ -3894,17 +3894,11 @@ int lsg_mlp_set_samples(lsg_mlp *m, int64_t n, const float *X, const float *T) {
   return 0;
 }
 
-static int mlpRows(int64_t count, int maxRows) {
-  int64_t r = (count + 63) / 64;
-  if (r > maxRows) r = maxRows;
-  return r < 1 ? 1 : (int)r;
-}
-
 int lsg_mlp_loss_grad(lsg_mlp *m, int64_t offset, int64_t count, double *loss, float *grad) {
   using namespace lsg;
   if (offset < 0 || count <= 0 || offset + count > m->n) return fail(-1, "lsg_mlp_loss_grad: sample range out of bounds");
   launchMlpGrad(g_ctx.s, m->X + offset * 8, m->T + offset, (uint32_t)count, m->P, m->partials,
-                mlpRows(count, m->rows), m->G);
+                mlpGradRows((uint32_t)count, m->rows), m->G);
   float h[MLP_PSTRIDE];
   LSG_HIP(hipMemcpyAsync(h, m->G, sizeof(h), hipMemcpyDeviceToHost, g_ctx.s));
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
@@ -3920,9 +3914,8 @@ int lsg_mlp_train(lsg_mlp *m, int iters, int64_t batch, double lr, double *lastL
   int64_t off = 0;
   for (int it = 0; it < iters; ++it) {
     if (off + batch > m->n) off = 0;
-    launchMlpGrad(g_ctx.s, m->X + off * 8, m->T + off, (uint32_t)batch, m->P, m->partials, mlpRows(batch, m->rows),
-                  m->G);
-    launchMlpAdam(g_ctx.s, m->P, m->M, m->V, m->G, ++m->step, (float)lr);
+    launchMlpGrad(g_ctx.s, m->X + off * 8, m->T + off, (uint32_t)batch, m->P, m->partials,
+                  mlpGradRows((uint32_t)batch, m->rows), m->G, m->M, m->V, ++m->step, (float)lr);
     off += batch;
   }
   if (lastLoss) {
