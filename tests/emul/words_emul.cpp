@@ -99,11 +99,7 @@ Words wordOp(const Words &in, double a, double b, const double *rates, double dt
     wordSite<D>(in.wb.data(), F, w, site);
     const int32_t kw = site.kw, yr = site.yr, zr = site.zr;
     const WordBits self = site.self;
-    if (star && quietSite<D>(F, site)) {
-      bool conflict = false;
-      check(starPoints<D, true>(in.wb.data(), F, w, site, conflict) == 0 && !conflict, "a quiet word has work");
-    }
-    const uint64_t cand = star ? starPoints<D, OP == W_EXPAND>(in.wb.data(), F, w, site, g_conflict) : self.def;
+    const uint64_t cand = star ? starPoints<D, OP == W_EXPAND>(F, site, g_conflict) : self.def;
     if (!cand) {
       check(self.def == 0, "a defined point is left out");
       o.wb[w] = self;
@@ -179,10 +175,10 @@ bool same(const EBand &x, const EBand &y) {
 extern "C" {
 
 // Runs operation `op` on the band of `h` both ways; 0 when the results are
-// the same bit for bit, 1 when not, 3 when not but a conflict was reported, -1
-// on a failed check.  `rates`: one value
-// per frame position (null: none); the number of positions comes back from a
-// call with op = -1.
+// the same bit for bit, 1 when not; 4 and 3 the same where a conflict was
+// reported; 2 when the conversions lose something; -1 on a failed check.
+// `rates`: one value per frame position (null: none); the number of positions
+// comes back from a call with op = -1.
 int64_t emu_words_compare(void *h, int op, double a, double b, const double *rates, double dt) {
   EBand &d = *(EBand *)h;
   if (op < 0) return 64 * (d.f.nwords + 1);
@@ -194,7 +190,7 @@ int64_t emu_words_compare(void *h, int op, double a, double b, const double *rat
     if (!same(toBand(in, d, d.width), d)) r = 2;
     else if (d.D == 2) r = same(toBand(runOp<2>(in, op, a, b, rates, dt), d, 0), listOp<2>(d, op, a, b, rates, dt)) ? 0 : 1;
     else r = same(toBand(runOp<3>(in, op, a, b, rates, dt), d, 0), listOp<3>(d, op, a, b, rates, dt)) ? 0 : 1;
-    if (r == 1 && g_conflict) r = 3;
+    if (g_conflict && (r == 0 || r == 1)) r = r == 1 ? 3 : 4;
   } catch (const std::exception &e) {
     fprintf(stderr, "words_emul: %s\n", e.what());
   }

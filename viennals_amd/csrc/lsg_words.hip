@@ -1,6 +1,6 @@
 // Kernels on word bands (lsg_words.hpp), written for CDNA4 (gfx950, wave64).
 //
-// One launch per band operation.  A workgroup takes strips of 16 words dealt
+// One launch per band operation.  A workgroup takes strips of words dealt
 // round robin over the grid, so that a slab of words with work (a flat part
 // of a surface fills whole layers of the frame) spreads over the chip.
 // First every thread looks at one word: the words with points to evaluate
@@ -20,13 +20,17 @@
 
 namespace lsg {
 
-static constexpr uint32_t STRIP = 16;
+// Strips of 8 words: the parts of a surface that fill whole rows come in runs
+// of words, and a workgroup with several full strips of 16 finished last
+// (trench 256, in us: PRUNE_RSZ 19.3 -> 17.2, UPD_REBUILD 35.4 -> 31.2); 4
+// words and less cost a large film its coalescing (film 1024: EXPAND 83.4 at
+// 8, 88.2 at 4, 96.5 at 2).
+static constexpr uint32_t STRIP = 8;
 
 __device__ inline uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ inline uint64_t uni(uint64_t v) { return (uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32); }
 
-// Workgroups of the word kernels: up to 16 strips (256 words, one per
-// thread) each, fewer while that gives 4 workgroups per CU.
+// Workgroups of the word kernels: up to 256 words (one per thread) each, fewer while that gives 4 workgroups per CU.
 static uint32_t wordGrid(uint32_t nw) {
   const uint32_t strips = (nw + STRIP - 1) / STRIP;
   const uint32_t per = std::max(1u, std::min((uint32_t)TPB / STRIP, strips / 1024u));
@@ -40,7 +44,7 @@ __device__ inline uint32_t xcdOrder(uint32_t b, uint32_t n) {
   return xcd * per + (xcd < rem ? xcd : rem) + k;
 }
 
-// The words of a workgroup in rounds of 16 strips (one word per thread);
+// The words of a workgroup in rounds of 256 (one word per thread);
 // thread-level `first(w, push)` decides whether word w goes on the list with
 // its 64-bit mask, wave-level `each(w, mask)` runs for every listed word.
 template <class First, class Each>
@@ -242,7 +246,7 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
       if (STAR) {
         wordSite<D>(wb, F, w, s);
         bool conflict = false;
-        if (!quietSite<D>(F, s)) cand = starPoints<D, OP == W_EXPAND>(wb, F, w, s, conflict);
+        cand = starPoints<D, OP == W_EXPAND>(F, s, conflict);
         if (OP == W_EXPAND && conflict) st->conflict = 1;
         listed = cand != 0;
         if (UPD && listed) {  // without an active point in its stars the word ends undefined

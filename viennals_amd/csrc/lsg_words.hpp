@@ -83,7 +83,6 @@ LSG_HD inline WordRef frameRef(const Frame &f, int32_t x, int32_t y, int32_t z) 
 struct WordFrame {
   Frame f;
   int32_t first[3], last[3];
-  int bounded0, periodic0;
   // the star of the grid-minimum entry: itself, then +1 and -1 along each
   // axis (word | bit << 24)
   uint32_t gmin[7];
@@ -97,8 +96,6 @@ struct WordFrame {
       if (a >= f.o[d] && a - f.o[d] < f.ext[d]) first[d] = a - f.o[d];
       if (b >= f.o[d] && b - f.o[d] < f.ext[d]) last[d] = b - f.o[d];
     }
-    bounded0 = g.bounded(0) ? 1 : 0;
-    periodic0 = g.bc[0] == PERIODIC ? 1 : 0;
     for (int k = 0; k < 7; ++k) {
       int32_t c[3] = {g.lo[0], g.lo[1], g.lo[2]};
       const int d = (k - 1) >> 1;
@@ -225,9 +222,6 @@ LSG_HD inline uint64_t startsOfWord(const WordBits *wb, const Frame &f, uint32_t
   const WordCarry c = w > 0 ? wordCarry(wb[w - 1], kw, f) : firstCarry(wb, f);
   return startBits(wb[w], c) & wordValid(f, kw);
 }
-LSG_HD inline uint64_t topStart(const WordBits &b) {  // whether bit 63 starts a run
-  return (b.def >> 63) | (b.def >> 62 & 1ull) | ((b.neg >> 63) ^ (b.neg >> 62 & 1ull));
-}
 
 // What the operations read around one word: its own bits, the words (or the
 // single points, WordRef) its points see a step away along y and z, and the
@@ -237,8 +231,6 @@ template <int D> struct WordSite {
   WordBits self;
   WordRef ref[2 * D - 2];   // [2 (d - 1)] a step +1 along axis d, [2 (d - 1) + 1] a step -1
   WordBits bits[2 * D - 2];
-  WordBits prev, prevs[2 * D - 2];  // the words before (of the row before at a row's start)
-  WordBits rowPrev;                 // periodic x: the word before the row
   WordRef below, above;
   int belowDef, belowNeg, aboveDef, aboveNeg;
 };
@@ -246,8 +238,6 @@ template <int D> LSG_HD inline void wordSite(const WordBits *wb, const WordFrame
   const Frame &f = F.f;
   f.wordRow(w, s.kw, s.yr, s.zr);
   s.self = wb[w];
-  s.prev = wb[w > 0 ? w - 1u : 0u];
-  if (F.periodic0) s.rowPrev = wb[w > (uint32_t)s.kw ? w - (uint32_t)s.kw - 1u : 0u];
   LSG_UNROLL
   for (int d = 1; d < D; ++d)
     LSG_UNROLL
@@ -255,7 +245,6 @@ template <int D> LSG_HD inline void wordSite(const WordBits *wb, const WordFrame
       const WordRef r = stepRef(F, w, s.yr, s.zr, d, k ? -1 : 1);
       s.ref[2 * d - 2 + k] = r;
       s.bits[2 * d - 2 + k] = wb[r.w];
-      s.prevs[2 * d - 2 + k] = wb[r.w > 0 ? r.w - 1u : 0u];
     }
   const int32_t row = s.zr * f.ext[1] + s.yr;
   s.below = edgeRef(F, w, s.kw, row, -1);
@@ -267,96 +256,42 @@ template <int D> LSG_HD inline void wordSite(const WordBits *wb, const WordFrame
   s.aboveNeg = (int)(p.neg >> s.above.bit & 1ull);
 }
 
-// Whether every point that starPoints looks at is undefined and of one sign:
-// the word then has no point to evaluate and no conflict.
-template <int D> LSG_HD inline bool quietSite(const WordFrame &F, const WordSite<D> &s) {
-  const uint64_t valid = wordValid(F.f, s.kw), neg = (s.self.neg & 1ull) ? valid : 0ull;
-  const int last = s.kw > 0 ? 63 : rowLastBit(F.f);
-  const int sign = (int)(s.self.neg & 1ull);
-  if (s.kw == 0 && s.yr == 0 && s.zr == 0) return false;  // the carry is the grid-minimum entry's
-  uint64_t any = s.self.def | (s.self.neg ^ neg) | (s.prev.def >> last & 1ull) | ((s.prev.neg >> last & 1ull) ^ (uint64_t)sign);
-  if (s.kw > 0) any |= (s.prev.def >> 62 & 1ull) | ((s.prev.neg >> 62 & 1ull) ^ (uint64_t)sign);
-  any |= (uint64_t)(s.belowDef | s.aboveDef | (s.belowNeg ^ sign) | (s.aboveNeg ^ sign));
-  if (F.periodic0) {  // the row's first point, which the last one sees
-    const int lb = rowLastBit(F.f);
-    any |= (s.rowPrev.def >> lb & 1ull) | ((s.rowPrev.neg >> lb & 1ull) ^ (uint64_t)sign);
-    if (s.yr == 0 && s.zr == 0) any |= 1ull;
-  }
-  LSG_UNROLL
-  for (int k = 0; k < 2 * D - 2; ++k) {
-    const WordBits Q = s.bits[k], Qp = s.prevs[k];
-    if (s.ref[k].bit >= 0) any |= (Q.def >> s.ref[k].bit & 1ull) | ((Q.neg >> s.ref[k].bit & 1ull) ^ (uint64_t)sign);
-    else any |= Q.def | (Q.neg ^ neg) | (Qp.def >> last & 1ull) | ((Qp.neg >> last & 1ull) ^ (uint64_t)sign);
-    if (s.ref[k].w == 0) any |= 1ull;
-  }
-  return any == 0ull;
-}
-
 // Points of word w at which a star operation has to be evaluated: those whose
-// boundary-mapped star holds a run start.  Every other point is undefined and
-// keeps its value.
+// boundary-mapped star holds a defined point.  Every other point is undefined
+// and keeps its value.
 //
-// The run-list pipeline (candStarWord) visits more points: the successors of
-// these and the first points of rows with a bounded x.  Their stars hold
-// undefined values only, so every rule returns the point's own value, except
-// the Expand rule where an undefined neighbour has the other sign: it then
-// changes the point, and in a run list all points after it up to the next
-// visited one.  Such fields (regions of opposite sign that touch without a
-// defined point) are not distance fields and have no word band counterpart:
-// `conflict` reports them, and the caller runs the operation on run lists.
+// The run-list pipeline (candStarWord) visits more points: those whose star
+// holds the start of an undefined run, the successors of all these and the
+// first points of rows with a bounded x.  Their stars hold undefined values
+// only, so every rule returns the point's own value, except the Expand rule
+// where an undefined neighbour has the other sign: it then changes the point,
+// and in a run list all points after it up to the next visited one.  Such
+// fields (regions of opposite sign that touch without a defined point) are
+// not distance fields and have no word band counterpart: `conflict` reports
+// every undefined point with such a neighbour, visited or not, and the caller
+// runs the operation on run lists.
 template <int D, bool CHECK>
-LSG_HD inline uint64_t starPoints(const WordBits *wb, const WordFrame &F, uint32_t w, const WordSite<D> &s,
-                                  bool &conflict) {
-  const Frame &f = F.f;
-  const int kw = s.kw, wl = wordLast(f), lb = rowLastBit(f);
+LSG_HD inline uint64_t starPoints(const WordFrame &F, const WordSite<D> &s, bool &conflict) {
   const WordBits B = s.self;
-  const WordBits P = s.prev;
-  const WordCarry carry = w > 0 ? wordCarry(P, kw, f) : firstCarry(wb, f);
-  const uint64_t valid = wordValid(f, kw);
-  const uint64_t S = startBits(B, carry) & valid;
-  uint64_t dil = S | (S << 1) | (S >> 1);
-  uint64_t prevTop = 0, mixed = 0;
-  if (kw > 0) {
-    const uint64_t s63 = topStart(P);
-    dil |= s63;
-    if (CHECK)
-      prevTop = s63 | (P.def >> 62 & 1ull) | (P.def >> 61 & 1ull) | ((P.neg >> 62 & 1ull) ^ (P.neg >> 61 & 1ull)) |
-                (S & 1ull);
-  }
-  if (kw < wl)  // the next word's first point
-    dil |= ((uint64_t)s.aboveDef | (B.def >> 63) | ((uint64_t)s.aboveNeg ^ (B.neg >> 63))) << 63;
-  if (F.periodic0) {
-    if (kw == wl) {  // the last point's +x neighbour is the row's first
-      const uint32_t w0 = w - (uint32_t)kw;
-      const WordCarry c0 = w0 > 0 ? wordCarry(s.rowPrev, 0, f) : firstCarry(wb, f);
-      if (startBits(wb[w0], c0) & 1ull) dil |= 1ull << lb;
-      if ((uint64_t)s.aboveNeg != (B.neg >> lb & 1ull)) mixed |= 1ull << lb;
-    }
-    if (kw == 0) {  // the first point's -x neighbour is the row's last
-      dil |= (uint64_t)s.belowDef;
-      mixed |= (uint64_t)s.belowNeg ^ (B.neg & 1ull);
-    }
-  }
+  const uint64_t valid = wordValid(F.f, s.kw), top = valid ^ (valid >> 1);
+  uint64_t c = B.def | (B.def << 1) | (B.def >> 1) | (uint64_t)s.belowDef | (s.aboveDef ? top : 0ull);
+  uint64_t mixed = 0;
+  if (CHECK)
+    mixed = (B.neg ^ ((B.neg << 1) | (uint64_t)s.belowNeg)) | (B.neg ^ ((B.neg >> 1) | (s.aboveNeg ? top : 0ull)));
   LSG_UNROLL
   for (int k = 0; k < 2 * D - 2; ++k) {
     const WordRef r = s.ref[k];
     const WordBits Q = s.bits[k];
     if (r.bit >= 0) {  // one point outside the frame's rows
       if (CHECK) mixed |= (Q.def >> r.bit & 1ull) ? ~0ull : (B.neg ^ ((Q.neg >> r.bit & 1ull) ? ~0ull : 0ull));
-      continue;
+    } else {
+      c |= Q.def;
+      if (CHECK) mixed |= B.neg ^ Q.neg;
     }
-    const WordBits Qp = s.prevs[k];
-    const WordCarry qc = r.w > 0 ? wordCarry(Qp, kw, f) : firstCarry(wb, f);
-    dil |= startBits(Q, qc) & valid;
-    mixed |= B.neg ^ Q.neg;
-    if (CHECK && kw > 0) prevTop |= topStart(Qp);
   }
-  dil &= valid;
-  if (CHECK) {
-    const uint64_t succ = (dil << 1) | prevTop | ((F.bounded0 && kw == 0) ? 1ull : 0ull);
-    if (succ & ~dil & mixed & valid) conflict = true;
-  }
-  return dil;
+  c &= valid;
+  if (CHECK && (mixed & valid & ~c)) conflict = true;
+  return c;
 }
 
 // Sign word of a boolean of two words without defined points (ruleBoolean on
