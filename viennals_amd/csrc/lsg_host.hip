@@ -2307,7 +2307,7 @@ static int advectApply(lsg_advect *a) {
   // steps on word bands: one level set with device-evaluated velocities and
   // nothing to do between the stages; the others read run lists
   bool words = !multi && wordBands(d) && !a->hostScalar && !a->hostVector && !a->saveVelocities && !a->ignoreVoids &&
-               !(a->velUpdate && a->temporal != 0) && a->spatial != 12;
+               !(a->velUpdate && a->temporal != 0) && (a->spatial != 12 || a->rp.learnedWave);
   auto prepareRuns = [&]() -> int {
     for (lsg_domain *l : a->levelSets) {
       if (int e = needRuns(l)) return e;

@@ -16,6 +16,7 @@
 #include <cstdint>
 
 #include "lsg_block.hpp"
+#include "lsg_mlp.hpp"
 #include "lsg_words_launch.hpp"
 
 namespace lsg {
@@ -509,20 +510,20 @@ void launchWordActive(hipStream_t s, const WordBufs &b, const Frame &f, uint64_t
 }
 
 // The active points of the workgroup's words, 256 words at a time, handed to
-// `fn` one per lane in full waves (the rest below a wave waits for the next
-// words), so that the scheme runs with idle lanes only once.  fn(p) gets the
-// frame position.  The list holds 64 words' worth of points; fuller rounds
-// run in parts.
+// all of its threads as lists of full waves (the rest below a wave waits for
+// the next words), so that the scheme runs with idle lanes only once.
+// fn(list, n) gets frame positions; the list is its until it returns.  The
+// list holds 64 words' worth of points; fuller rounds run in parts.
 static constexpr uint32_t ACTIVE_LIST = 4096;
 // words dealt to the workgroups in pairs: the words of a flat part of the
 // surface are full and lie side by side, and a strip of 16 of them would be
 // 16 waves of work for one workgroup beside workgroups with one
 static constexpr uint32_t PAIR = 2;
 template <class Fn>
-__device__ __attribute__((always_inline)) inline void forActivePoints(const uint64_t *__restrict__ act, uint32_t nw,
+__device__ __attribute__((always_inline)) inline void forActiveLists(const uint64_t *__restrict__ act, uint32_t nw,
                                                                       uint32_t b, uint32_t nb, Fn fn) {
   __shared__ uint32_t list[ACTIVE_LIST + 64];
-  const uint32_t lane = threadIdx.x & 63u, wid = threadIdx.x >> 6;
+  const uint32_t lane = threadIdx.x & 63u;
   const uint32_t pairs = (nw + PAIR - 1) / PAIR;
   uint32_t held = 0;  // points left from the round before, at the list's start
   for (uint32_t j0 = 0; j0 * nb + b < pairs; j0 += TPB / PAIR) {
@@ -550,7 +551,7 @@ __device__ __attribute__((always_inline)) inline void forActivePoints(const uint
       __syncthreads();
       const uint32_t n = held + part;
       const uint32_t take = last ? n : n / 64u * 64u;
-      for (uint32_t i = wid * 64u + lane; i < take; i += TPB) fn(list[i]);
+      if (take) fn(list, take);
       __syncthreads();
       held = n - take;
       uint32_t p = 0;
@@ -562,6 +563,15 @@ __device__ __attribute__((always_inline)) inline void forActivePoints(const uint
       if (done >= total) break;
     }
   }
+}
+
+// The same one point per thread: fn(p).
+template <class Fn>
+__device__ __attribute__((always_inline)) inline void forActivePoints(const uint64_t *__restrict__ act, uint32_t nw,
+                                                                      uint32_t b, uint32_t nb, Fn fn) {
+  forActiveLists(act, nw, b, nb, [&](const uint32_t *list, uint32_t n) {
+    for (uint32_t i = threadIdx.x; i < n; i += TPB) fn(list[i]);
+  });
 }
 
 __device__ inline void blockMaxSlot(double v, unsigned long long *slots) {
@@ -581,9 +591,38 @@ __global__ __launch_bounds__(256) void kWordAlphas(WordView v, const uint64_t *_
   for (int d = 0; d < D; ++d) blockMaxSlot(la[d], st->alpha[stage][d]);
 }
 
+// The terms of one axis of a wave's points with the learned weights (phase 1
+// and 2 of weno5LearnedAxes); `rows` are the wave's 128 rows of network inputs.
+__device__ __attribute__((always_inline)) inline AxisTerms learnedTerms(const WordView &v, uint32_t p,
+                                                                        const int32_t r[3], int d, double phi0,
+                                                                        bool on, float *rows, const MlpLane &W) {
+  float *io = rows + 2 * MLP_IN * (threadIdx.x & 63u);
+  AxisTerms t{0., 0., 0.};
+  double st[1][7];
+  if (on) {
+    axisValues<1, 3>(v, p, r, d, st[0]);
+    st[0][3] = phi0;
+    t.c = st[0][4] - st[0][2];
+    weno5LearnedAxes<1>(st, v.g.dx, nullptr, io, &t.m, &t.q, 1);
+  } else {
+    for (int q = 0; q < 2 * MLP_IN; ++q) io[q] = 0.f;
+  }
+  waveSyncLds();
+  waveMlp<128>(rows, W);
+  if (on) weno5LearnedAxes<1>(st, v.g.dx, nullptr, io, &t.m, &t.q, 2);
+  waveSyncLds();  // the rows are rewritten by the next points
+  return t;
+}
+
 // Advect::integrateTime for one level set (lsAdvect.hpp:495-593): the stage
 // velocity of every active point at its slot of `rates`, the maxima in the
 // step's slots.
+//
+// A workgroup has few active points (20 to 100 where the frame is small or
+// the chip just filled), so its time is the chain of one point's loads and
+// divisions.  The axes of a point are therefore dealt to the four waves, 64
+// points and one axis at a time, and a lane combines the terms of its point
+// from LDS.
 template <int D, int SCHEME>
 __global__ __launch_bounds__(256) void kWordRates(WordView v, const uint64_t *__restrict__ act, uint32_t nw,
                                                   RateParams rp, double *__restrict__ rates,
@@ -594,16 +633,67 @@ __global__ __launch_bounds__(256) void kWordRates(WordView v, const uint64_t *__
     for (int d = 0; d < D; ++d) ga[d] = slotMax(st->alpha[stage][d]);
   double lmax = 0.;
   unsigned long long points = 0, key = 0;
-  forActivePoints(act, nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](uint32_t p) {
-    ++points;
-    double velocity;
-    bool used = false, outside = false;
-    rates[p] = wordRatePoint<D, SCHEME>(v, p, rp, vel, ga, la, velocity, used, box, &outside);
-    if (SCHEME == S_LLF_BOX && outside) st->conflict = 1;
-    if (SCHEME == S_SLLF && used && (unsigned long long)p + 1ull > key) key = (unsigned long long)p + 1ull;
-    const double m = fabs(velocity);
-    if (lmax < m) lmax = m;
-  });
+  if constexpr (axisScheme(SCHEME)) {
+    constexpr bool LEARNED = SCHEME == S_WENO5L;
+    __shared__ double terms[3 * D][TPB];
+    __shared__ float rows[LEARNED ? TPB * 2 * MLP_IN : 1];
+    MlpLane W;
+    if constexpr (LEARNED) W = mlpLane(rp.mlp);
+    forActiveLists(act, nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](const uint32_t *list, uint32_t n) {
+      const uint32_t lane = threadIdx.x & 63u;
+      const int wave = (int)uni(threadIdx.x >> 6);
+      for (uint32_t g = 0; g < n; g += TPB) {
+        const uint32_t m = n - g < (uint32_t)TPB ? n - g : (uint32_t)TPB;
+        const int tasks = (int)((m + 63u) / 64u) * D;
+        for (int q = wave; q < tasks; q += TPB / 64) {
+          const int d = q % D;
+          const uint32_t i = (uint32_t)(q / D) * 64u + lane;
+          const bool on = i < m;
+          if (!LEARNED && !on) continue;
+          const uint32_t p = list[on ? g + i : g];
+          int32_t r[3];
+          v.f.decode(p, r[0], r[1], r[2]);
+          const double phi0 = v.val[p];
+          AxisTerms t;
+          if constexpr (LEARNED) t = learnedTerms(v, p, r, d, phi0, on, rows + wave * 128 * MLP_IN, W);
+          else t = axisTerms<SCHEME>(v, p, r, d, phi0, rp.order);
+          if (on) {
+            terms[3 * d][i] = t.m;
+            terms[3 * d + 1][i] = t.q;
+            terms[3 * d + 2][i] = t.c;
+          }
+        }
+        __syncthreads();
+        if (threadIdx.x < m) {
+          AxisTerms t[D];
+          LSG_UNROLL
+          for (int d = 0; d < D; ++d)
+            t[d] = AxisTerms{terms[3 * d][threadIdx.x], terms[3 * d + 1][threadIdx.x], terms[3 * d + 2][threadIdx.x]};
+          const uint32_t p = list[g + threadIdx.x];
+          ++points;
+          double velocity;
+          bool outside = false;
+          rates[p] = combineTerms<D, SCHEME>(v, p, t, rp, vel, ga, la, velocity, box, &outside);
+          if (SCHEME == S_LLF_BOX && outside) st->conflict = 1;
+          const double a = fabs(velocity);
+          if (lmax < a) lmax = a;
+        }
+        __syncthreads();
+      }
+    });
+  } else {
+    forActivePoints(act, nw, xcdOrder(blockIdx.x, gridDim.x), gridDim.x, [&](uint32_t p) {
+      ++points;
+      double velocity;
+      bool used = false;
+      int32_t c[3];
+      v.coords(p, c);
+      rates[p] = ratePoint<D, SCHEME>(v, c, v.val[p], rp, vel, ga, la, velocity, nullptr, nullptr, &used);
+      if (SCHEME == S_SLLF && used && (unsigned long long)p + 1ull > key) key = (unsigned long long)p + 1ull;
+      const double m = fabs(velocity);
+      if (lmax < m) lmax = m;
+    });
+  }
   blockMaxSlot(lmax, st->maxAbs[stage]);
   if (SCHEME == S_LLLF || SCHEME == S_LLF || SCHEME == S_LLFA || SCHEME == S_LLF_BOX)
     for (int d = 0; d < D; ++d) blockMaxSlot(la[d], st->alpha[stage][d]);
@@ -725,6 +815,7 @@ static void wordRates(hipStream_t s, const WordView &v, const uint64_t *act, uin
   switch (schemeIdOf(rp.spatial)) {
   case S_EO: LSG_WR(S_EO); break;
   case S_WENO5: LSG_WR(S_WENO5); break;
+  case S_WENO5L: LSG_WR(S_WENO5L); break;
   case S_LF: LSG_WR(S_LF); break;
   case S_LLLF: LSG_WR(S_LLLF); break;
   case S_LLFA: LSG_WR(S_LLFA); break;

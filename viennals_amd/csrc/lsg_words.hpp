@@ -378,11 +378,12 @@ LSG_HD inline double wordRuleMin(const WordFrame &F, const WordBits *wb, const d
 }
 
 // ------------------------------------------------------------- schemes ----
-// The one-dimensional schemes of lsg_items.hpp (same expressions, same order
-// of operations) with one pass of a rolled loop per axis: the code of a
-// kernel stays small enough for the instruction cache, which a workgroup
-// that evaluates one or two waves of points otherwise fills from memory, and
-// one axis' values are in flight at a time.
+// The schemes of lsg_items.hpp (same expressions, same order of operations)
+// in two parts: the terms of one axis (axisTerms) and the point's velocity
+// from the terms of all (combineTerms).  Different waves take the axes of a
+// point, and the code of the first part is there once, not once per axis: a
+// workgroup that evaluates one or two waves of points otherwise spends its
+// time filling the instruction cache.
 
 // Values at distance K0 .. K along axis d of point p (frame coordinates r,
 // absolute c): st[K + k] = phi(c + k e_d).  Every point is a slot at a fixed
@@ -423,193 +424,137 @@ LSG_HD inline void axisValues(const WordView &v, uint32_t p, const int32_t r[3],
   }
 }
 
-// One double per axis with an index that is not a constant.
-struct Axes {
-  double v[3] = {0., 0., 0.};
-  LSG_HD void set(int d, double x) {
-    v[0] = d == 0 ? x : v[0];
-    v[1] = d == 1 ? x : v[1];
-    v[2] = d == 2 ? x : v[2];
-  }
+// Terms of one axis.  WENO: the two one-sided derivatives and the central
+// difference of the normal; otherwise the differences to the point before and
+// after (upwindDiffs) and their mean at distance 1.
+struct AxisTerms {
+  double m, q, c;
 };
-
-// schemeWENO
-template <int D, int ORDER>
-LSG_HD inline RateOut wordWENO(const WordView &b, uint32_t p, const int32_t r[3], double phi0, bool calcNormals,
-                               const Vel &vel) {
-  constexpr int R = (ORDER + 1) / 2;
-  double gradPosTotal = 0, gradNegTotal = 0, denominator = 0;
-  Axes gm, gp, n;
-#if defined(__clang__)
-#pragma unroll 1
-#endif
-  for (int d = 0; d < D; ++d) {
+template <int SCHEME>
+LSG_HD inline AxisTerms axisTerms(const WordView &b, uint32_t p, const int32_t r[3], int d, double phi0, int order) {
+  AxisTerms t;
+  if (SCHEME == S_WENO3 || SCHEME == S_WENO5) {
+    constexpr int R = SCHEME == S_WENO5 ? 3 : 2;
     double st[2 * R + 1];
     axisValues<1, R>(b, p, r, d, st);
     st[R] = phi0;
-    const double cd = st[R + 1] - st[R - 1];
-    double m, q;
-    if (ORDER == 3) {
-      m = weno3(st, b.g.dx, false);
-      q = weno3(st, b.g.dx, true);
+    t.c = st[R + 1] - st[R - 1];
+    if (SCHEME == S_WENO3) {
+      t.m = weno3(st, b.g.dx, false);
+      t.q = weno3(st, b.g.dx, true);
     } else {
-      m = weno5(st, b.g.dx, false);
-      q = weno5(st, b.g.dx, true);
+      t.m = weno5(st, b.g.dx, false);
+      t.q = weno5(st, b.g.dx, true);
     }
-    gradPosTotal += pow2(dmaxs(m, 0.0)) + pow2(dmins(q, 0.0));
-    gradNegTotal += pow2(dmins(m, 0.0)) + pow2(dmaxs(q, 0.0));
-    gm.set(d, m);
-    gp.set(d, q);
-    if (calcNormals) {
-      n.set(d, cd);
-      denominator += cd * cd;
-    }
-  }
-  if (calcNormals && denominator > 0) {
-    denominator = 1. / sqrt(denominator);
-    LSG_UNROLL
-    for (int i = 0; i < D; ++i) n.v[i] *= denominator;
-  }
-  double vel_grad = 0.;
-  const double sv = vel.scalar(n.v);
-  if (sv > 0) vel_grad += sqrt(gradPosTotal) * sv;
-  else vel_grad += sqrt(gradNegTotal) * sv;
-  LSG_UNROLL
-  for (int w = 0; w < D; w++) {
-    if (vel.vec[w] > 0.) vel_grad += vel.vec[w] * gm.v[w];
-    else vel_grad += vel.vec[w] * gp.v[w];
-  }
-  return {vel_grad, 0.};
-}
-
-// One-sided differences of every axis (gatherUpwind, upwindDiffs): pos[d] =
-// diffNeg, neg[d] = diffPos as the schemes name their gradients; `each(d,
-// diffPos, diffNeg, centred)` accumulates, centred = ((phi+ - phi0) + (phi0 -
-// phi-)) / 2.
-template <int D, class Each>
-LSG_HD inline void wordUpwind(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order, Axes &pos,
-                              Axes &neg, Each each) {
-#if defined(__clang__)
-#pragma unroll 1
-#endif
-  for (int d = 0; d < D; ++d) {
+  } else {
     double st[5], s1[3];
     axisValues<1, 1>(b, p, r, d, s1);
     st[0] = st[4] = 0.;
     if (order == 2) axisValues<2, 2>(b, p, r, d, st);
     st[1] = s1[0];
     st[3] = s1[2];
-    double diffPos, diffNeg;
-    upwindDiffs(st, b.g.dx, order, phi0, diffPos, diffNeg);
-    pos.set(d, diffNeg);
-    neg.set(d, diffPos);
-    each(d, diffPos, diffNeg, ((st[3] - phi0) + (phi0 - st[1])) * 0.5);
+    upwindDiffs(st, b.g.dx, order, phi0, t.q, t.m);
+    t.c = ((st[3] - phi0) + (phi0 - st[1])) * 0.5;
   }
+  return t;
 }
 
-// schemeEO
-template <int D>
-LSG_HD inline RateOut wordEO(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
-                             bool calcNormals, const Vel &vel) {
-  Axes pos, neg, n;
-  double gradPosTotal = 0, gradNegTotal = 0, denominator = 0;
-  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double centred) {
-    gradPosTotal += pow2(dmaxs(diffNeg, 0.0)) + pow2(dmins(diffPos, 0.0));
-    gradNegTotal += pow2(dmins(diffNeg, 0.0)) + pow2(dmaxs(diffPos, 0.0));
-    if (calcNormals) {
-      n.set(d, centred);
-      denominator += centred * centred;
-    }
-  });
-  if (calcNormals) {
-    denominator = 1. / sqrt(denominator);
-    LSG_UNROLL
-    for (int i = 0; i < D; ++i) n.v[i] *= denominator;
-  }
-  double vel_grad = 0.;
-  const double sv = vel.scalar(n.v);
-  if (sv > 0) vel_grad += sqrt(gradPosTotal) * sv;
-  else vel_grad += sqrt(gradNegTotal) * sv;
+// The last part of every scheme: the vector velocity upwind.
+template <int D> LSG_HD inline double addVector(const AxisTerms *t, const Vel &vel, double g) {
   LSG_UNROLL
   for (int w = 0; w < D; w++) {
-    if (vel.vec[w] > 0.) vel_grad += vel.vec[w] * pos.v[w];
-    else vel_grad += vel.vec[w] * neg.v[w];
+    if (vel.vec[w] > 0.) g += vel.vec[w] * t[w].m;
+    else g += vel.vec[w] * t[w].q;
   }
-  return {vel_grad, 0.};
+  return g;
+}
+
+// schemeEO, schemeWENO (only the latter guards a vanishing gradient).
+template <int D, bool GUARD> LSG_HD inline RateOut combineEO(const AxisTerms *t, bool calcNormals, const Vel &vel) {
+  double gradPosTotal = 0, gradNegTotal = 0, denominator = 0;
+  double n[3] = {0., 0., 0.};
+  LSG_UNROLL
+  for (int d = 0; d < D; ++d) {
+    gradPosTotal += pow2(dmaxs(t[d].m, 0.0)) + pow2(dmins(t[d].q, 0.0));
+    gradNegTotal += pow2(dmins(t[d].m, 0.0)) + pow2(dmaxs(t[d].q, 0.0));
+    if (calcNormals) {
+      n[d] = t[d].c;
+      denominator += t[d].c * t[d].c;
+    }
+  }
+  if (calcNormals && (!GUARD || denominator > 0)) {
+    denominator = 1. / sqrt(denominator);
+    LSG_UNROLL
+    for (int i = 0; i < D; ++i) n[i] *= denominator;
+  }
+  double vel_grad = 0.;
+  const double sv = vel.scalar(n);
+  if (sv > 0) vel_grad += sqrt(gradPosTotal) * sv;
+  else vel_grad += sqrt(gradNegTotal) * sv;
+  return {addVector<D>(t, vel, vel_grad), 0.};
 }
 
 // schemeLF
 template <int D>
-LSG_HD inline RateOut wordLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
-                             bool calcNormals, const Vel &vel, double alphaFactor, const double *alphas) {
-  Axes pos, neg, n;
+LSG_HD inline RateOut combineLF(const AxisTerms *t, bool calcNormals, const Vel &vel, double alphaFactor,
+                                const double *alphas) {
+  double n[3] = {0., 0., 0.};
   double grad = 0., dissipation = 0., modulus = 0.;
-  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double) {
-    const double m = (diffNeg + diffPos) * 0.5;
+  LSG_UNROLL
+  for (int d = 0; d < D; ++d) {
+    const double m = (t[d].m + t[d].q) * 0.5;
     if (calcNormals) {
-      n.set(d, m);
+      n[d] = m;
       modulus += m * m;
     }
     grad += pow2(m);
-    const double alpha = d == 0 ? alphas[0] : (d == 1 ? alphas[1] : alphas[2]);
-    dissipation += alphaFactor * alpha * (diffPos - diffNeg) * 0.5;
-  });
+    dissipation += alphaFactor * alphas[d] * (t[d].q - t[d].m) * 0.5;
+  }
   if (calcNormals) {
     modulus = 1. / sqrt(modulus);
     LSG_UNROLL
-    for (int i = 0; i < D; ++i) n.v[i] *= modulus;
+    for (int i = 0; i < D; ++i) n[i] *= modulus;
   }
-  const double sv = vel.scalar(n.v);
+  const double sv = vel.scalar(n);
   double totalGrad = 0.;
   if (sv != 0.) totalGrad = sv * sqrt(grad);
-  LSG_UNROLL
-  for (int w = 0; w < D; w++) {
-    if (vel.vec[w] > 0.) totalGrad += vel.vec[w] * pos.v[w];
-    else totalGrad += vel.vec[w] * neg.v[w];
-  }
+  totalGrad = addVector<D>(t, vel, totalGrad);
   return {totalGrad, (totalGrad != 0.) ? dissipation : 0};
 }
 
 // The gradient part that schemeLLLF and schemeLLF share: the total gradient
 // and the normalised centred gradient.
-template <int D>
-LSG_HD inline double wordLocalGradient(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
-                                       const Vel &vel, Axes &pos, Axes &neg, Axes &n, double &sv) {
+template <int D> LSG_HD inline double localGradient(const AxisTerms *t, const Vel &vel, double n[3], double &sv) {
   double grad = 0., modulus = 0.;
-  wordUpwind<D>(b, p, r, phi0, order, pos, neg, [&](int d, double diffPos, double diffNeg, double) {
-    const double m = (diffNeg + diffPos) * 0.5;
-    n.set(d, m);
+  LSG_UNROLL
+  for (int d = 0; d < D; ++d) {
+    const double m = (t[d].m + t[d].q) * 0.5;
+    n[d] = m;
     modulus += m * m;
     grad += pow2(m);
-  });
+  }
   modulus = 1. / sqrt(modulus);
   LSG_UNROLL
-  for (int i = 0; i < D; ++i) n.v[i] *= modulus;
-  sv = vel.scalar(n.v);
+  for (int i = 0; i < D; ++i) n[i] *= modulus;
+  sv = vel.scalar(n);
   double totalGrad = 0.;
   if (sv != 0.) totalGrad = sv * sqrt(grad);
-  LSG_UNROLL
-  for (int w = 0; w < D; w++) {
-    if (vel.vec[w] > 0.) totalGrad += vel.vec[w] * pos.v[w];
-    else totalGrad += vel.vec[w] * neg.v[w];
-  }
-  return totalGrad;
+  return addVector<D>(t, vel, totalGrad);
 }
 
 // schemeLLLF
 template <int D>
-LSG_HD inline RateOut wordLLLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
-                               const Vel &vel, double alphaFactor, double *alphaAcc) {
-  Axes pos, neg, n;
+LSG_HD inline RateOut combineLLLF(const AxisTerms *t, const Vel &vel, double alphaFactor, double *alphaAcc) {
+  double n[3] = {0., 0., 0.};
   double sv;
-  const double totalGrad = wordLocalGradient<D>(b, p, r, phi0, order, vel, pos, neg, n, sv);
+  const double totalGrad = localGradient<D>(t, vel, n, sv);
   if (totalGrad == 0.) return {0., 0.};
   double dissipation = 0.;
   LSG_UNROLL
   for (int i = 0; i < D; ++i) {
-    const double alpha = fabs((sv + vel.vec[i]) * n.v[i]);
+    const double alpha = fabs((sv + vel.vec[i]) * n[i]);
     alphaAcc[i] = dmaxs(alphaAcc[i], alpha);
-    dissipation += alphaFactor * alpha * (neg.v[i] - pos.v[i]) * 0.5;
+    dissipation += alphaFactor * alpha * (t[i].q - t[i].m) * 0.5;
   }
   return {totalGrad, dissipation};
 }
@@ -660,11 +605,12 @@ template <int D> LSG_HD inline size_t boxSlot(uint32_t p, int k) {
 // schemeLLF with the box alphas of the band's points at hand; `outside` is
 // set where a box point lies outside the frame (nothing is read there).
 template <int D>
-LSG_HD inline RateOut wordLLF(const WordView &b, uint32_t p, const int32_t r[3], double phi0, int order,
-                              const Vel &vel, double alphaFactor, double *alphaAcc, const double *box, bool &outside) {
-  Axes pos, neg, n;
+LSG_HD inline RateOut combineLLF(const WordView &b, uint32_t p, const int32_t r[3], const AxisTerms *terms,
+                                 const Vel &vel, double alphaFactor, double *alphaAcc, const double *box,
+                                 bool &outside) {
+  double n[3] = {0., 0., 0.};
   double sv;
-  const double totalGrad = wordLocalGradient<D>(b, p, r, phi0, order, vel, pos, neg, n, sv);
+  const double totalGrad = localGradient<D>(terms, vel, n, sv);
   if (totalGrad == 0.) return {0., 0.};
   // slot offsets of the steps -1, 0, +1 along each axis
   int32_t off[3][3] = {{0, 0, 0}, {0, 0, 0}, {0, 0, 0}};
@@ -708,7 +654,7 @@ LSG_HD inline RateOut wordLLF(const WordView &b, uint32_t p, const int32_t r[3],
   LSG_UNROLL
   for (int i = 0; i < D; ++i) {
     alphaAcc[i] = fmax(alphaAcc[i], alpha[i]);
-    dissipation += alphaFactor * alpha[i] * (neg.v[i] - pos.v[i]) * 0.5;
+    dissipation += alphaFactor * alpha[i] * (terms[i].q - terms[i].m) * 0.5;
   }
   return {totalGrad, dissipation};
 }
@@ -717,25 +663,26 @@ LSG_HD inline RateOut wordLLF(const WordView &b, uint32_t p, const int32_t r[3],
 // word kernels beside SchemeId's).
 constexpr int S_LLF_BOX = 16;
 
-// ratePoint for an active point of a word band.
+// Whether a scheme runs in the two parts; the others look their points up one
+// by one (ratePoint).
+LSG_HD constexpr bool axisScheme(int scheme) {
+  return scheme == S_EO || scheme == S_WENO3 || scheme == S_WENO5 || scheme == S_WENO5L || scheme == S_LF ||
+         scheme == S_LLLF || scheme == S_LLF_BOX;
+}
+// ratePoint for an active point of a word band from the terms of its axes.
 template <int D, int SCHEME>
-LSG_HD inline double wordRatePoint(const WordView &v, uint32_t p, const RateParams &rp, const Vel &vel,
-                                   const double *globalAlphas, double *alphaAcc, double &velocity, bool &sllfUsed,
-                                   const double *box = nullptr, bool *outside = nullptr) {
-  int32_t r[3];
-  v.f.decode(p, r[0], r[1], r[2]);
-  const double phi0 = v.val[p];
+LSG_HD inline double combineTerms(const WordView &v, uint32_t p, const AxisTerms *t, const RateParams &rp,
+                                  const Vel &vel, const double *globalAlphas, double *alphaAcc, double &velocity,
+                                  const double *box = nullptr, bool *outside = nullptr) {
   RateOut o;
-  if (SCHEME == S_EO) o = wordEO<D>(v, p, r, phi0, rp.order, rp.calcNormals != 0, vel);
-  else if (SCHEME == S_WENO5) o = wordWENO<D, 5>(v, p, r, phi0, rp.calcNormals != 0, vel);
-  else if (SCHEME == S_WENO3) o = wordWENO<D, 3>(v, p, r, phi0, rp.calcNormals != 0, vel);
-  else if (SCHEME == S_LF) o = wordLF<D>(v, p, r, phi0, rp.order, rp.calcNormals != 0, vel, rp.alphaFactor, globalAlphas);
-  else if (SCHEME == S_LLLF) o = wordLLLF<D>(v, p, r, phi0, rp.order, vel, rp.alphaFactor, alphaAcc);
-  else if (SCHEME == S_LLF_BOX) o = wordLLF<D>(v, p, r, phi0, rp.order, vel, rp.alphaFactor, alphaAcc, box, *outside);
-  else {
-    const int32_t c[3] = {r[0] + v.f.o[0], r[1] + v.f.o[1], r[2] + v.f.o[2]};
-    return ratePoint<D, SCHEME>(v, c, phi0, rp, vel, globalAlphas, alphaAcc, velocity, nullptr, nullptr, &sllfUsed);
-  }
+  if (SCHEME == S_EO) o = combineEO<D, false>(t, rp.calcNormals != 0, vel);
+  else if (SCHEME == S_LF) o = combineLF<D>(t, rp.calcNormals != 0, vel, rp.alphaFactor, globalAlphas);
+  else if (SCHEME == S_LLLF) o = combineLLLF<D>(t, vel, rp.alphaFactor, alphaAcc);
+  else if (SCHEME == S_LLF_BOX) {
+    int32_t r[3];
+    v.f.decode(p, r[0], r[1], r[2]);
+    o = combineLLF<D>(v, p, r, t, vel, rp.alphaFactor, alphaAcc, box, *outside);
+  } else o = combineEO<D, true>(t, rp.calcNormals != 0, vel);
   velocity = o.H - o.Dn;
   double x = velocity;
   if ((rp.checkDissipation && (o.H < 0 && x > 0)) || (o.H > 0 && x < 0)) x = 0;
