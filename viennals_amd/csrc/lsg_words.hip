@@ -14,6 +14,8 @@
 
 #include <algorithm>
 #include <cstdint>
+#include <mutex>
+#include <unordered_map>
 
 #include "lsg_block.hpp"
 #include "lsg_mlp.hpp"
@@ -31,11 +33,31 @@ static constexpr uint32_t STRIP = 8;
 __device__ inline uint32_t uni(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
 __device__ inline uint64_t uni(uint64_t v) { return (uint64_t)uni((uint32_t)v) | ((uint64_t)uni((uint32_t)(v >> 32)) << 32); }
 
-// Workgroups of the word kernels: up to 256 words (one per thread) each, fewer while that gives 4 workgroups per CU.
-static uint32_t wordGrid(uint32_t nw) {
-  const uint32_t strips = (nw + STRIP - 1) / STRIP;
-  const uint32_t per = std::max(1u, std::min((uint32_t)TPB / STRIP, strips / 1024u));
-  return (strips + per - 1) / per;
+// Workgroups of `kernel` that the chip holds at once.
+static uint32_t residentBlocks(const void *kernel) {
+  static std::mutex m;
+  static std::unordered_map<const void *, uint32_t> known;
+  std::lock_guard<std::mutex> lock(m);
+  uint32_t &n = known[kernel];
+  if (!n) {
+    int perCu = 0, cus = 0, dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&perCu, kernel, TPB, 0) != hipSuccess || perCu * cus <= 0)
+      perCu = 4, cus = 256;
+    n = (uint32_t)(perCu * cus);
+  }
+  return n;
+}
+// Workgroups of a word kernel, `extra` of them beside those that take words:
+// as many as run at once, each with up to 256 words (one per thread); for more
+// words a multiple of that.  A few workgroups over the resident number would
+// wait for the first to end and double the kernel's time: with 1057 on 1024
+// places, half of EXPAND's 12.2 us on a sphere of 80 cells was their wait.
+static uint32_t wordGrid(const void *kernel, uint32_t nw, uint32_t extra = 0) {
+  const uint32_t strips = (nw + STRIP - 1) / STRIP, room = residentBlocks(kernel);
+  const uint32_t turns = (uint32_t)(((uint64_t)nw + extra + (uint64_t)room * TPB - 1) / ((uint64_t)room * TPB));
+  return std::min(strips + extra, std::max(1u, turns) * room);
 }
 
 // XCD-contiguous index of worker block b of n.
@@ -179,7 +201,7 @@ __device__ inline double laneOf(double v, int l) {
 // words of a round are dealt to the waves (record i to wave i % 4); a wave
 // keeps its records in registers, one per lane, and reads them lane by lane.
 template <int D> struct WordRecords {
-  uint32_t word[TPB];            // last valid bit | ONE_POINT
+  uint32_t word[TPB];            // last valid bit | ONE_POINT | HAS_RATES ..
   uint32_t self[TPB];            // byte offset of the word's slots
   uint32_t ref[2 * D - 2][TPB];  // of the neighbour words' slots (ONE_POINT words: | 1 where one point is meant)
   uint32_t end[2][TPB];          // of the slots below the first and above the last point
@@ -188,6 +210,9 @@ template <int D> struct WordRecords {
   uint32_t count;
 };
 static constexpr uint32_t ONE_POINT = 256u;
+// UPD_REBUILD: record bits of the slots that may hold active points (and so
+// rates): the word itself, its neighbours, the points below and above
+static constexpr uint32_t HAS_RATES = 512u;
 
 // One band operation.  Workgroup 0 evaluates the grid-minimum entry and, in
 // a step's first operation, resets the step's scalars; the others take the
@@ -240,6 +265,7 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
     const uint32_t strip = (j0 + threadIdx.x / STRIP) * nb + b;
     const uint32_t w = strip * STRIP + threadIdx.x % STRIP;
     uint64_t cand = 0;
+    uint32_t rated = 0;
     bool listed = false;
     WordSite<D> s;
     uint64_t valid = ~0ull;
@@ -251,12 +277,13 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
         if (OP == W_EXPAND && conflict) st->conflict = 1;
         listed = cand != 0;
         if (UPD && listed) {  // without an active point in its stars the word ends undefined
-          uint64_t act = a.inAct[w];
+          rated = a.inAct[w] ? HAS_RATES : 0u;
           LSG_UNROLL
-          for (int k = 0; k < NR; ++k) act |= s.ref[k].w < nw ? a.inAct[s.ref[k].w] : 1ull;
-          act |= s.below.w < nw ? a.inAct[s.below.w] : 1ull;
-          act |= s.above.w < nw ? a.inAct[s.above.w] : 1ull;
-          if (!act) {
+          for (int k = 0; k < NR; ++k)
+            if (s.ref[k].w < nw ? a.inAct[s.ref[k].w] : 1ull) rated |= HAS_RATES << (1 + k);
+          if (s.below.w < nw ? a.inAct[s.below.w] >> s.below.bit & 1ull : 1ull) rated |= HAS_RATES << (NR + 1);
+          if (s.above.w < nw ? a.inAct[s.above.w] >> s.above.bit & 1ull : 1ull) rated |= HAS_RATES << (NR + 2);
+          if (!rated) {
             const uint64_t neg = s.self.neg;
             s.self = WordBits{0, neg};
             valid = wordValid(f, s.kw);
@@ -286,7 +313,7 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
       if (listed) {
         const uint32_t i = at + (uint32_t)__builtin_popcountll(has & ((1ull << lane) - 1ull));
         valid = wordValid(f, s.kw);
-        uint32_t word = s.kw == wordLast(f) ? (uint32_t)rowLastBit(f) : 63u;
+        uint32_t word = (s.kw == wordLast(f) ? (uint32_t)rowLastBit(f) : 63u) | rated;
         R.self[i] = wordOffset(w);
         R.cand[i] = cand;
         // the input's slots: of the word itself they are the operation's
@@ -330,7 +357,7 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
       }
       uint32_t dLo = 0, dHi = 0, nLo = 0, nHi = 0, aLo = 0, aHi = 0;  // results, record j in lane j
       struct Star {
-        double v[2 * D];
+        double v[2 * D], r[UPD ? 2 * D : 1];
       };
       auto at = [&](uint32_t x, uint32_t j) { return (uint32_t)__builtin_amdgcn_readlane((int)x, (int)j); };
       auto put = [&](uint32_t j, double o) {
@@ -364,25 +391,26 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
           z.v[2 * D - 1] = slotAt(val, lane < 32u ? e0 : e1);
         }
       };
-      auto update = [&](uint32_t j, Star &z) {  // updateLevelSet's rule on the star
-        auto one = [&](double v, uint32_t off) {
-          const bool act = fabs(v) <= 0.5;
-          double r = 0.;
-          if (__any(act)) r = slotAt(rates, off);
-          return ruleUpdate(v, dt, r);
-        };
-        z.v[0] = one(z.v[0], at(rIn, j) + lane8);
-        const bool single = at(rWord, j) & ONE_POINT;
+      // the rates of the star, from a page where there are none: all loads of
+      // a star in flight together
+      auto loadRates = [&](uint32_t j, Star &z) {
+        const uint32_t word = at(rWord, j);
+        z.r[0] = slotAt(rates, ((word & HAS_RATES) ? at(rIn, j) : 0u) + lane8);
         LSG_UNROLL
         for (int k = 0; k < NR; ++k) {
-          const uint32_t o = at(rRef[k], j);
-          z.v[1 + k] = one(z.v[1 + k], (single && (o & 1u)) ? (o & ~7u) : (o & ~7u) + lane8);
+          const uint32_t o = (word & (HAS_RATES << (1 + k))) ? at(rRef[k], j) : 0u;
+          z.r[1 + k] = slotAt(rates, (o & ~7u) + ((o & 1u) ? 0u : lane8));
         }
-        const uint32_t e0 = at(rEnd[0], j), e1 = at(rEnd[1], j);
-        z.v[2 * D - 1] = one(z.v[2 * D - 1], lane < 32u ? e0 : e1);
+        const uint32_t e0 = (word & (HAS_RATES << (NR + 1))) ? at(rEnd[0], j) : 0u;
+        const uint32_t e1 = (word & (HAS_RATES << (NR + 2))) ? at(rEnd[1], j) : 0u;
+        z.r[2 * D - 1] = slotAt(rates, lane < 32u ? e0 : e1);
+      };
+      auto update = [&](Star &z) {  // updateLevelSet's rule on the star
+        LSG_UNROLL
+        for (int k = 0; k < 2 * D; ++k) z.v[k] = ruleUpdate(z.v[k], dt, z.r[k]);
       };
       auto finish = [&](uint32_t j, Star &z) {
-        if (UPD) update(j, z);
+        if (UPD) update(z);
         const double c = z.v[0];
         const uint64_t c64 = (uint64_t)at((uint32_t)rCand, j) | ((uint64_t)at((uint32_t)(rCand >> 32), j) << 32);
         double nbv[2 * D];
@@ -404,7 +432,9 @@ __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb
         const uint32_t k = j + 1 < mine ? j + 1 : j;  // the last of an odd number twice, with the same result
         Star x, y;
         load(j, x);
+        if (UPD) loadRates(j, x);
         load(k, y);
+        if (UPD) loadRates(k, y);
         finish(j, x);
         finish(k, y);
       }
@@ -429,11 +459,10 @@ template <int D>
 static void wordStar(hipStream_t s, int op, const WordBufs &in, const WordBufs &out, const Frame &f, const GridInfo &g,
                      const WordOpArgs &a, WordStep *st) {
   const uint32_t nw = (uint32_t)f.nwords;
-  const uint32_t grid = wordGrid(nw) + 1;
   WordFrame F;
   F.init(f, g);
 #define LSG_WORD(OP) \
-  kWordStar<D, OP><<<grid, TPB, 0, s>>>(in.wb, in.val, a.rates, out.wb, out.val, a.act, F, g, nw, a, st)
+  kWordStar<D, OP><<<wordGrid((const void *)kWordStar<D, OP>, nw, 1), TPB, 0, s>>>(in.wb, in.val, a.rates, out.wb, out.val, a.act, F, g, nw, a, st)
   switch (op) {
   case W_EXPAND: LSG_WORD(W_EXPAND); break;
   case W_REBUILD: LSG_WORD(W_REBUILD); break;
@@ -482,7 +511,7 @@ __global__ __launch_bounds__(256) void kWordBool(const WordBits *__restrict__ aw
 void launchWordBoolean(hipStream_t s, const WordBufs &A, const WordBufs &B, const WordBufs &out, const Frame &f,
                        int kind, double wTarget, double wSource) {
   const uint32_t nw = (uint32_t)f.nwords;
-  kWordBool<<<wordGrid(nw + 1), TPB, 0, s>>>(A.wb, A.val, B.wb, B.val, out.wb, out.val, f, nw, kind, wTarget, wSource);
+  kWordBool<<<wordGrid((const void *)kWordBool, nw + 1), TPB, 0, s>>>(A.wb, A.val, B.wb, B.val, out.wb, out.val, f, nw, kind, wTarget, wSource);
 }
 
 // ------------------------------------------------------------- rates ----
@@ -506,7 +535,7 @@ __global__ __launch_bounds__(256) void kWordActive(const WordBits *__restrict__ 
 }
 void launchWordActive(hipStream_t s, const WordBufs &b, const Frame &f, uint64_t *act) {
   const uint32_t nw = (uint32_t)f.nwords;
-  kWordActive<<<wordGrid(nw), TPB, 0, s>>>(b.wb, b.val, act, nw);
+  kWordActive<<<wordGrid((const void *)kWordActive, nw), TPB, 0, s>>>(b.wb, b.val, act, nw);
 }
 
 // The active points of the workgroup's words, 256 words at a time, handed to
@@ -795,8 +824,8 @@ template <int D> __global__ void kWordSllfAlphas(WordView v, RateParams rp, int 
 }
 
 // Workgroups of the passes over active points: 256 words each from 4 per CU on.
-static uint32_t activeGrid(uint32_t nw) {
-  return std::min(4096u, std::max(std::min(1024u, (nw + PAIR - 1) / PAIR), (nw + TPB - 1) / TPB));
+static uint32_t activeGrid(uint32_t nw, uint32_t most = 4096u) {
+  return std::min(most, std::max(std::min(1024u, (nw + PAIR - 1) / PAIR), (nw + TPB - 1) / TPB));
 }
 
 void launchWordAlphas(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
@@ -815,7 +844,9 @@ static void wordRates(hipStream_t s, const WordView &v, const uint64_t *act, uin
   switch (schemeIdOf(rp.spatial)) {
   case S_EO: LSG_WR(S_EO); break;
   case S_WENO5: LSG_WR(S_WENO5); break;
-  case S_WENO5L: LSG_WR(S_WENO5L); break;
+  case S_WENO5L:  // as many workgroups as their registers let run together
+    kWordRates<D, S_WENO5L><<<activeGrid(nw, 512u), TPB, 0, s>>>(v, act, nw, rp, rates, box, stage, count, st);
+    break;
   case S_LF: LSG_WR(S_LF); break;
   case S_LLLF: LSG_WR(S_LLLF); break;
   case S_LLFA: LSG_WR(S_LLFA); break;
@@ -823,7 +854,7 @@ static void wordRates(hipStream_t s, const WordView &v, const uint64_t *act, uin
     if (box) {
       WordFrame F;
       F.init(v.f, v.g);
-      kWordBoxAlphas<D><<<wordGrid(nw), TPB, 0, s>>>(v, act, F, nw, rp, box);
+      kWordBoxAlphas<D><<<wordGrid((const void *)kWordBoxAlphas<D>, nw), TPB, 0, s>>>(v, act, F, nw, rp, box);
       LSG_WR(S_LLF_BOX);
     } else {
       LSG_WR(S_LLF);
@@ -873,7 +904,7 @@ __global__ __launch_bounds__(256) void kWordImport(const uint64_t *__restrict__ 
 }
 void launchWordImport(hipStream_t s, const BandBufs &in, const WordBufs &out, const Frame &f) {
   const uint32_t nw = (uint32_t)f.nwords;
-  kWordImport<<<wordGrid(nw), TPB, 0, s>>>(in.bits, in.pre, in.val, out.wb, out.val, f, nw);
+  kWordImport<<<wordGrid((const void *)kWordImport, nw), TPB, 0, s>>>(in.bits, in.pre, in.val, out.wb, out.val, f, nw);
 }
 
 // Canonical run list of a word band, in two kernels over contiguous chunks:
@@ -967,7 +998,7 @@ __global__ __launch_bounds__(256) void kWordCopy(const WordBits *__restrict__ wb
 }
 void launchWordCopy(hipStream_t s, const WordBufs &in, const WordBufs &out, const Frame &f) {
   const uint32_t nw = (uint32_t)f.nwords;
-  kWordCopy<<<wordGrid(nw + 1), TPB, 0, s>>>(in.wb, in.val, out.wb, out.val, f, nw);
+  kWordCopy<<<wordGrid((const void *)kWordCopy, nw + 1), TPB, 0, s>>>(in.wb, in.val, out.wb, out.val, f, nw);
 }
 
 __global__ __launch_bounds__(256) void kWordReframe(WordView v, WordBits *__restrict__ owb, double *__restrict__ oval,
@@ -988,7 +1019,7 @@ __global__ __launch_bounds__(256) void kWordReframe(WordView v, WordBits *__rest
 void launchWordReframe(hipStream_t s, const WordBufs &in, const Frame &f, const GridInfo &g, const WordBufs &out,
                        const Frame &fo) {
   const uint32_t nwo = (uint32_t)fo.nwords;
-  kWordReframe<<<wordGrid(nwo), TPB, 0, s>>>(WordView{in.wb, in.val, f, g}, out.wb, out.val, fo, nwo);
+  kWordReframe<<<wordGrid((const void *)kWordReframe, nwo), TPB, 0, s>>>(WordView{in.wb, in.val, f, g}, out.wb, out.val, fo, nwo);
 }
 
 __global__ void kWordStatsInit(uint32_t *count, int32_t *bbox, const WordStep *st, uint32_t *conflict) {
@@ -1069,7 +1100,7 @@ __global__ __launch_bounds__(256) void kWordNegate(WordBits *__restrict__ wb, do
 }
 void launchWordNegate(hipStream_t s, const WordBufs &b, const Frame &f) {
   const uint32_t nw = (uint32_t)f.nwords;
-  kWordNegate<<<wordGrid(nw + 1), TPB, 0, s>>>(b.wb, b.val, f, nw);
+  kWordNegate<<<wordGrid((const void *)kWordNegate, nw + 1), TPB, 0, s>>>(b.wb, b.val, f, nw);
 }
 
 }  // namespace lsg
