@@ -595,30 +595,54 @@ static int needRuns(lsg_domain *d, bool mayAllocate = true) {
   return fail(-40, "band capacity overflow");
 }
 
-static int downloadRuns(lsg_domain *d, std::vector<int32_t> &idx, std::vector<double> &val) {
+// Grid indices of a run list's entries, D each: decoded here, so that the
+// arrays go to the caller's memory as they are (decoded on the host from the
+// positions, through two arrays of its own, a list of 5M entries took 9 ms).
+static __global__ void kRunIndices(const uint32_t *pos, uint32_t n, Frame f, GridInfo g, int D, int32_t *idx) {
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+    int32_t r[3];
+    if (i == 0 && f.base) {  // the grid-minimum entry
+      for (int k = 0; k < 3; ++k) r[k] = g.lo[k];
+    } else {
+      f.decode(pos[i], r[0], r[1], r[2]);
+      for (int k = 0; k < 3; ++k) r[k] += f.o[k];
+    }
+    for (int k = 0; k < D; ++k) idx[(size_t)i * D + k] = r[k];
+  }
+}
+
+// The run list into memory that `room(n, idx, val)` names for its n entries.
+template <class Room> static int downloadRuns(lsg_domain *d, Room room) {
   if (int e = ctxInit()) return e;
   if (int e = needRuns(d)) return e;
   uint32_t n = 0;
   LSG_HIP(hipMemcpyAsync(&n, d->cur.b.n, sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
   LSG_HIP(hipStreamSynchronize(g_ctx.s));
-  std::vector<uint32_t> pos(n);
-  val.resize(n);
-  LSG_HIP(hipMemcpyAsync(val.data(), d->cur.b.val, n * sizeof(double), hipMemcpyDeviceToHost, g_ctx.s));
-  LSG_HIP(hipMemcpyAsync(pos.data(), d->cur.b.pos, n * sizeof(uint32_t), hipMemcpyDeviceToHost, g_ctx.s));
-  LSG_HIP(hipStreamSynchronize(g_ctx.s));
-  const int D = d->D;
-  idx.resize((size_t)n * D);
-  for (uint32_t i = 0; i < n; ++i) {
-    if (i == 0 && d->f.base) {
-      for (int k = 0; k < D; ++k) idx[k] = d->g.lo[k];
-      continue;
-    }
-    int32_t r[3];
-    d->f.decode(pos[i], r[0], r[1], r[2]);
-    for (int k = 0; k < D; ++k) idx[(size_t)i * D + k] = r[k] + d->f.o[k];
+  int32_t *idx = nullptr;
+  double *val = nullptr;
+  if (int e = room((size_t)n, idx, val)) return e;
+  if (n) {
+    const size_t bytes = (size_t)n * d->D * sizeof(int32_t);
+    int32_t *di = nullptr;
+    LSG_HIP(devMalloc(&di, bytes));
+    kRunIndices<<<std::min<uint32_t>(4096u, (n + 255u) / 256u), 256, 0, g_ctx.s>>>(d->cur.b.pos, n, d->f, d->g, d->D, di);
+    hipError_t e = hipMemcpyAsync(val, d->cur.b.val, n * sizeof(double), hipMemcpyDeviceToHost, g_ctx.s);
+    if (e == hipSuccess) e = hipMemcpyAsync(idx, di, bytes, hipMemcpyDeviceToHost, g_ctx.s);
+    if (e == hipSuccess) e = hipStreamSynchronize(g_ctx.s);
+    (void)devFree(di);
+    LSG_HIP(e);
   }
   d->hostN = n;
   return 0;
+}
+static int downloadRuns(lsg_domain *d, std::vector<int32_t> &idx, std::vector<double> &val) {
+  return downloadRuns(d, [&](size_t n, int32_t *&i, double *&v) {
+    idx.resize(n * d->D);
+    val.resize(n);
+    i = idx.data();
+    v = val.data();
+    return 0;
+  });
 }
 
 static bool idxLessD(int D, const int32_t *a, const int32_t *b) {
@@ -3444,13 +3468,12 @@ int lsg_mark_void_points(lsg_domain *d) {
 }
 
 int lsg_domain_get_runs(lsg_domain *d, int32_t *idx, double *val, int64_t cap) {
-  std::vector<int32_t> ri;
-  std::vector<double> rv;
-  if (int e = downloadRuns(d, ri, rv)) return e;
-  if ((int64_t)rv.size() > cap) return fail(-1, "buffer too small");
-  std::memcpy(idx, ri.data(), ri.size() * sizeof(int32_t));
-  std::memcpy(val, rv.data(), rv.size() * sizeof(double));
-  return 0;
+  return downloadRuns(d, [&](size_t n, int32_t *&i, double *&v) {
+    if ((int64_t)n > cap) return fail(-1, "buffer too small");
+    i = idx;
+    v = val;
+    return 0;
+  });
 }
 
 int lsg_domain_num_points(lsg_domain *d, int64_t *n) {
