@@ -867,13 +867,13 @@ static void wordRates(hipStream_t s, const WordView &v, const uint64_t *act, uin
 }
 void launchWordRates(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
                      const uint64_t *act, double *rates, double *box, int stage, int count, WordStep *st,
-                     hipEvent_t e0, hipEvent_t e1, bool externalEvents) {
+                     hipEvent_t e0, hipEvent_t e1) {
   const WordView v{b.wb, b.val, f, g};
   const uint32_t nw = (uint32_t)f.nwords;
-  if (e0) (void)hipEventRecordWithFlags(e0, s, externalEvents ? hipEventRecordExternal : hipEventRecordDefault);
+  if (e0) (void)hipEventRecord(e0, s);
   if (D == 2) wordRates<2>(s, v, act, nw, rp, rates, box, stage, count, st);
   else wordRates<3>(s, v, act, nw, rp, rates, box, stage, count, st);
-  if (e1) (void)hipEventRecordWithFlags(e1, s, externalEvents ? hipEventRecordExternal : hipEventRecordDefault);
+  if (e1) (void)hipEventRecord(e1, s);
   if (schemeIdOf(rp.spatial) == S_SLLF) {
     if (D == 2) kWordSllfAlphas<2><<<1, 1, 0, s>>>(v, rp, stage, st);
     else kWordSllfAlphas<3><<<1, 1, 0, s>>>(v, rp, stage, st);

@@ -63,7 +63,7 @@ void launchWordAlphas(hipStream_t s, int D, const WordBufs &b, const Frame &f, c
 void launchWordRates(hipStream_t s, int D, const WordBufs &b, const Frame &f, const GridInfo &g, const RateParams &rp,
                      const uint64_t *act, double *rates, double *box, int stage, int count, WordStep *st,
                      hipEvent_t e0 = nullptr,
-                     hipEvent_t e1 = nullptr, bool externalEvents = false);
+                     hipEvent_t e1 = nullptr);
 // Canonical run list <-> word band.
 void launchWordImport(hipStream_t s, const BandBufs &in, const WordBufs &out, const Frame &f);
 void launchWordExport(hipStream_t s, const WordBufs &in, BandBufs &out, const Frame &f, const GridInfo &g,
