@@ -10,7 +10,7 @@ value = point-updates/s: active points (|phi| <= 0.5) summed over the RK
 stages of the K timed steps, divided by the wall time of those steps with
 the band resident in HBM.  Two kernels of the step are then timed with HIP
 events on the library's stream over K more steps: the rule evaluation of
-the star band operations (Expand cycles and rebuilds; kEvalKeep<EvalStar>,
+the star band operations (Expand cycles and rebuilds; kWordStar,
 algorithmic bytes 8 B per input entry and 8 B per candidate; with
 --single-pass the whole single-pass operation kBandOp<AtStar>, 12 B per
 input entry read and per output entry written, value and position, plus
@@ -212,7 +212,7 @@ def sequential(vls, seq_sets, vels, W, R3, steps):
 
 
 def measured_traffic(kernel, workload):
-    """HBM bytes per launch of `kernel` (file tag: kRates, kBandOpStar) from
+    """HBM bytes per launch of `kernel` (file tag: kWordRates, kWordStar) from
     the committed rocprofv3 FETCH_SIZE / WRITE_SIZE summary of this workload
     (scaled by the copy-kernel calibration), or None."""
     path = os.path.join(ROOT, "profiles", f"{kernel}_{workload}_traffic.md")
@@ -348,9 +348,9 @@ def main():
         star = roofline("kBandOpStar", "kBandOp<AtStar> (single-pass Expand / rebuild band operation)",
                         adv.getStarKernelStats())
     else:
-        star = roofline("kEvalKeepStar", "kEvalKeep<EvalStar> (Expand / rebuild rule evaluation)",
-                        adv.getStarKernelStats())
-    rate = roofline("kRates", "kRates (Hamiltonian + CFL reduction)", adv.getRateKernelStats())
+        star = roofline("kWordStar", "kWordStar (Expand / rebuild on word bands)", adv.getStarKernelStats())
+    rate = (roofline("kRates", "kRates (Hamiltonian + CFL reduction)", adv.getRateKernelStats()) if single_pass else
+            roofline("kWordRates", "kWordRates (Hamiltonian + CFL reduction)", adv.getRateKernelStats()))
     measured = [star, rate]
     if not single_pass:
         measured.append(roofline("kEvalKeepStar2", "kEvalKeep<EvalStar2> (two Expand cycles at once)",

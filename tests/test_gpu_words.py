@@ -1,0 +1,103 @@
+"""Steps and band operations on word bands (64-point words of the frame)
+against the oracle, bit for bit, at the sizes where a word, a row or a strip
+of words ends, over the boundary conditions, and where the run list has to
+take over."""
+import numpy as np
+import pytest
+
+import cases
+import pyoracle as po
+from test_gpu_parity import _advect_gpu, assert_same, say, to_gpu
+
+pytestmark = pytest.mark.gpu
+
+REF, INF, PER = cases.REF, cases.INF, cases.PER
+
+
+def surface(nx, ny, bx, by):
+    """A gentle surface z = h(x, y) over nx * ny points (slopes up to 1/2, so
+    that a layer of points on each side of it is defined)."""
+    gmin, gmax = [0, 0, -60], [nx - (bx == REF), ny - (by == REF), 60]
+    d = po.Domain(3, gmin, gmax, [bx, by, INF], 1.0)
+    x, y = np.meshgrid(np.arange(nx), np.arange(ny), indexing="ij")
+    h = 0.3 + 0.04 * min(nx, 40) * np.cos(2 * np.pi * x / nx) + 0.04 * min(ny, 40) * np.cos(2 * np.pi * y / ny)
+    pts, vals = [], []
+    for z in range(-6, 8):
+        phi = (z - h) / 1.2
+        m = np.abs(phi) <= 1
+        pts.append(np.stack([x[m], y[m], np.full(m.sum(), z)], 1))
+        vals.append(phi[m])
+    d.from_points(np.concatenate(pts).astype(np.int32), np.concatenate(vals), 2)
+    return d
+
+
+def step(o, spatial, temporal, vel, time, tag):
+    g = to_gpu(o)
+    p = po.make_params(spatial=spatial, temporal=temporal, cfl=0.4, time=time, vel=vel)
+    st, r = po.advect(o, p)
+    assert st == 0
+    a = _advect_gpu(g, p)
+    assert a.getNumberOfTimeSteps() == r["steps"]
+    assert a.getAdvectedTime() == r["advected_time"]
+    assert a.getPointUpdates() == r["point_updates"]
+    assert_same(o, g, tag)
+
+
+@pytest.mark.parametrize("nx,ny,bx,by", [(1, 9, REF, PER), (2, 2, REF, REF), (63, 5, REF, REF), (64, 4, PER, REF),
+                                         (65, 7, REF, PER), (127, 3, PER, PER), (128, 17, REF, REF),
+                                         (200, 33, PER, PER)])
+@pytest.mark.parametrize("spatial,temporal", [(0, 0), (3, 1), (6, 1), (8, 2), (10, 2), (11, 2)])
+def test_steps_at_word_edges(nx, ny, bx, by, spatial, temporal):
+    say(f"words: advect {nx}x{ny} bc {bx},{by} spatial={spatial} temporal={temporal}")
+    step(surface(nx, ny, bx, by), spatial, temporal, cases.VEL_NORMAL_SQ, 1.2, "word edges")
+
+
+@pytest.mark.parametrize("vel", [cases.VEL_GROW, cases.VEL_NORMAL_SQ,
+                                 dict(kind=1, dir=0, k=1, b=0.1, a_pos=1.0, a_neg=0.3),
+                                 dict(kind=0, b=0.3, vec=(0.4, -0.2, 0.1))])
+@pytest.mark.parametrize("bx", [REF, PER])
+def test_local_alphas_of_the_box(vel, bx):
+    """The box alphas are shared between points except where a mirror changes
+    the speed (a speed by the sign of n_x on a reflective x axis)."""
+    say(f"words: LLF2 bc {bx} vel {vel}")
+    step(surface(70, 20, bx, REF), 8, 2, vel, 1.2, "box alphas")
+
+
+@pytest.mark.parametrize("temporal", [0, 2])
+def test_a_surface_that_leaves_its_frame(temporal):
+    say("words: 30 cells of etching, temporal %d" % temporal)
+    step(surface(66, 6, REF, REF), 0, temporal, dict(kind=0, b=-1.0), 30.0, "re-framed")
+
+
+def test_operations_to_the_frame_edge_and_back():
+    say("words: expand to 41 layers, reduce, prune, rebuild")
+    import viennals_amd as vls
+    o = surface(65, 5, PER, REF)
+    g = to_gpu(o)
+    for w in (9, 41):
+        o.expand(w)
+        vls.Expand(g, w).apply()
+        assert_same(o, g, f"expand {w}")
+    o.reduce(3)
+    vls.Reduce(g, 3).apply()
+    assert_same(o, g, "reduce")
+    o.prune(False)
+    vls.Prune(g).apply()
+    assert_same(o, g, "prune")
+
+
+def test_touching_undefined_regions_go_to_the_run_list():
+    """Undefined regions of opposite sign side by side, no defined point
+    between them: Expand reports them and runs on the run list."""
+    say("words: undefined regions of opposite sign")
+    import viennals_amd as vls
+    big = np.finfo(np.float64).max
+    o = po.Domain(3, [0, 0, -60], [70, 10, 60], [REF, REF, INF], 1.0)
+    idx = np.array([[0, 0, -60], [10, 4, 0], [11, 4, 0], [40, 4, 0], [20, 7, 2], [21, 7, 2]], np.int32)
+    val = np.array([big, 0.25, -big, big, -0.5, big])
+    idx[0] = [0, 0, int(o.get()[0][0][2])]
+    o.set(idx, val, 2)
+    g = to_gpu(o)
+    o.expand(4)
+    vls.Expand(g, 4).apply()
+    assert_same(o, g, "touching regions")

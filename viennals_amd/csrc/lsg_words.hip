@@ -218,9 +218,17 @@ static constexpr uint32_t HAS_RATES = 512u;
 // a step's first operation, resets the step's scalars; the others take the
 // words.
 //
-// The cost of a word is its instructions (about 100, a quarter of them the
+// The cost of a word is its instructions (about 90, a quarter of them the
 // rule) and one round of 2 D loads; two words are in flight per wave.  A word
 // without points to evaluate costs its share of the first phase only.
+// Measured, with the five launches on the run list it replaces (us), for a
+// trench of 256^2 and a film of 1024^2: EXPAND 13.0 and 85 (44 and 250),
+// UPD_REBUILD 23.5 and 143 (52 and 420).  At 1024^2 it moves the full 512-byte
+// words of which a third is defined.  Tried: a cheap test for words far from
+// the surface before the look at their neighbours (EXPAND 13.9 and 89: another
+// barrier and round trip), and slabs of rows per XCD so that neighbouring
+// layers meet in one L2 (the step of the trench 1.5 times as long: its walls
+// lie in two of the slabs).
 template <int D, int OP>
 __global__ __launch_bounds__(256) void kWordStar(const WordBits *__restrict__ wb, const double *__restrict__ val,
                                                  const double *__restrict__ rates, WordBits *__restrict__ owb,
@@ -546,7 +554,8 @@ void launchWordActive(hipStream_t s, const WordBufs &b, const Frame &f, uint64_t
 static constexpr uint32_t ACTIVE_LIST = 4096;
 // words dealt to the workgroups in pairs: the words of a flat part of the
 // surface are full and lie side by side, and a strip of 16 of them would be
-// 16 waves of work for one workgroup beside workgroups with one
+// 16 waves of work for one workgroup beside workgroups with one (WENO5 on a
+// trench of 256^2: 44 us in strips of 16, 30 in pairs)
 static constexpr uint32_t PAIR = 2;
 template <class Fn>
 __device__ __attribute__((always_inline)) inline void forActiveLists(const uint64_t *__restrict__ act, uint32_t nw,
@@ -651,7 +660,9 @@ __device__ __attribute__((always_inline)) inline AxisTerms learnedTerms(const Wo
 // the chip just filled), so its time is the chain of one point's loads and
 // divisions.  The axes of a point are therefore dealt to the four waves, 64
 // points and one axis at a time, and a lane combines the terms of its point
-// from LDS.
+// from LDS.  Against a lane that goes through its axes (us): EO, sphere of 80
+// cells 22.4 -> 9.4; WENO5, trench of 256^2 28.6 -> 17.6; WENO3, film of
+// 333 x 217 24.0 -> 11.1.
 template <int D, int SCHEME>
 __global__ __launch_bounds__(256) void kWordRates(WordView v, const uint64_t *__restrict__ act, uint32_t nw,
                                                   RateParams rp, double *__restrict__ rates,
@@ -743,7 +754,8 @@ __global__ __launch_bounds__(256) void kWordRates(WordView v, const uint64_t *__
 
 // Box alphas (boxAlphas) of every point in the 3^D box of an active point, in
 // words: computed once per point here where the scheme's own loop computes
-// the normal of each of the 3^D box points of every active point.
+// the normal of each of the 3^D box points of every active point.  A stage of
+// a film of 1024^2: 150 us here and 155 in the rate kernel, 531 without.
 template <int D>
 __global__ __launch_bounds__(256) void kWordBoxAlphas(WordView v, const uint64_t *__restrict__ act, WordFrame F,
                                                       uint32_t nw, RateParams rp, double *__restrict__ box) {
